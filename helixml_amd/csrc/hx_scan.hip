@@ -23,6 +23,7 @@
 
 #include "hx_common.h"
 #include "hx_wave.h"
+#include "hx_scan_ps.h"
 
 namespace hx {
 namespace {
@@ -1004,7 +1005,6 @@ __device__ inline void buf_store(float v, __amdgpu_buffer_rsrc_t rs, uint32_t of
 __device__ inline void buf_store(float v, __amdgpu_buffer_rsrc_t rs, uint32_t off, uint16_t*) {
     __builtin_amdgcn_raw_buffer_store_b16(Storage<uint16_t>::round(v), rs, off, 0, kStream);
 }
-constexpr int kBufRsrcWord3 = 0x00020000;  // gfx9 raw buffer: 32-bit data format, no swizzle
 
 // ----------------------------------------------------------------------------- warp-specialised
 // A block of 4 waves owns 48 channels of one batch row, and its waves have different jobs:
@@ -1733,6 +1733,7 @@ struct ScanArgs {
     hipStream_t stream;
     void* ws = nullptr;      // caller workspace for the segmented long-sequence path (nullable:
     size_t ws_bytes = 0;     // without one the sequence is never segmented)
+    bool ws_may_be_short = false;  // the workspace is a buffer that happens to be free: use what fits
 };
 
 // Time segments of the wave path: only when the (batch, 64-channel tile) pairs alone cannot fill
@@ -1759,6 +1760,84 @@ size_t scan_seg_bytes(int64_t Bt, int64_t Dm, int64_t nseg) {
     if (nseg <= 1) return 0;
     const size_t per = (size_t)Bt * Dm * 16;
     return (size_t)nseg * 3 * per * sizeof(float);
+}
+
+// Time segments of scan_ps_kernel for Bt x Dm channels. At most 128 (batch, 64-channel) tiles leave
+// half of the 256 CUs idle, and cutting the sequence costs a second, cheaper pass over it (1.75 times
+// the work at most): worth it from there. One block per CU measured best (24 tiles x 2048 steps: 34 us
+// against 38 with two and 126 uncut; 48 tiles x 1021 bf16 steps 33, 36 and 78), two where one leaves a
+// third of the CUs idle (128 tiles x 1000 steps: 61 us against 67) or segments past 4096 steps, whose
+// end-state passes stop early (32 tiles x 65536 steps: 600 us against 640). At least 64 steps each,
+// none below 512, at most sqrt(L) of them: the output pass starts with a latency-bound chain over the
+// segments before its own, and a launch costs about 5 us.
+int64_t ps_segments(int64_t Bt, int64_t Dm, int64_t L) {
+    const int64_t pairs = ((Dm + 63) / 64) * Bt;
+    if (g_scan_segments > 0) return g_scan_segments;
+    if (pairs > 128 || L < 512) return 1;
+    int64_t nseg = 256 / pairs;
+    if (pairs > 85 || L > 4096 * nseg) nseg = 512 / pairs;
+    if (nseg > L / 64) nseg = L / 64;
+    while (nseg > 1 && nseg * nseg > L) --nseg;
+    return nseg;
+}
+// Segment length (16-step aligned) and the count it gives.
+int64_t ps_seg_len(int64_t L, int64_t nseg) { return ((L + nseg - 1) / nseg + 15) / 16 * 16; }
+int64_t ps_seg_count(int64_t L, int64_t seg_len) { return (L + seg_len - 1) / seg_len; }
+// Scratch: every segment's end state and decay but the last's.
+size_t ps_seg_bytes(int64_t Bt, int64_t Dm, int64_t nseg) {
+    if (nseg <= 1) return 0;
+    return (size_t)(nseg - 1) * 2 * Bt * ((Dm + 63) / 64) * 64 * 16 * sizeof(float);
+}
+size_t ps_workspace_bytes(int64_t Bt, int64_t Dm, int64_t L) {
+    return ps_seg_bytes(Bt, Dm, ps_seg_count(L, ps_seg_len(L, ps_segments(Bt, Dm, L))));
+}
+// scan_ps_kernel's sizes: a segment's byte offsets, a few chunks of read-ahead included, below 2^31.
+bool ps_ok(int64_t Bt, int64_t Dm, int64_t L, size_t es) {
+    return L < (1LL << 30) && (L + 96) * Dm * (int64_t)es < (1LL << 31) && Bt * ((Dm + 63) / 64) <= 0x7fffffff;
+}
+
+template <typename T, bool HAS_Z, bool SP, int DTPK>
+int launch_ps(const ScanArgs& a, const uint16_t* dtlo, const uint16_t* wdt) {
+    const int64_t ntiles = (a.Dm + 63) / 64;
+    int64_t nseg = 1;
+    if (a.ws) {
+        nseg = ps_segments(a.Bt, a.Dm, a.L);
+        const size_t need = ps_workspace_bytes(a.Bt, a.Dm, a.L);
+        if (a.ws_bytes < need || !aligned(a.ws, 16)) {
+            // a workspace too small for a long sequence is refused; elsewhere as many segments as fit
+            HX_REQUIRE(g_scan_segments == 0 && (a.L < 4096 || a.ws_may_be_short), HX_ERR_INVALID_INPUT,
+                       "selective scan: workspace of %zu bytes (16-byte aligned) needed, %zu given "
+                       "(hx_selective_scan_workspace_size)", need, a.ws_bytes);
+            nseg = aligned(a.ws, 16) ? 1 + (int64_t)(a.ws_bytes / ps_seg_bytes(a.Bt, a.Dm, 2)) : 1;
+        }
+    }
+    const int64_t seg_len = ps_seg_len(a.L, nseg);
+    nseg = ps_seg_count(a.L, seg_len);
+    HX_REQUIRE(ntiles * a.Bt * nseg <= 0x7fffffff, HX_ERR_UNSUPPORTED,
+               "selective scan: %lld blocks exceed the grid", (long long)(ntiles * a.Bt * nseg));
+    float4* hend = (float4*)a.ws;
+    float4* decay = hend + (nseg - 1) * a.Bt * ntiles * 256;
+    const PsArgs pa{a.L, a.Dm, (int)ntiles, (int)a.Bt, (int)nseg, (int)seg_len, a.A, a.D, a.dt_bias,
+                    a.init_state, a.last_state, hend, decay, dtlo, wdt};
+    if (nseg > 1) {
+        hipLaunchKernelGGL((scan_ps_kernel<T, false, SP, true, DTPK>), dim3((unsigned)(ntiles * a.Bt * (nseg - 1))),
+                           dim3(512), 0, a.stream, pa, (const T*)a.u, (const T*)a.delta, (const T*)a.B,
+                           (const T*)nullptr, (const T*)nullptr, (T*)nullptr);
+        HX_LAUNCH_CHECK();
+    }
+    hipLaunchKernelGGL((scan_ps_kernel<T, HAS_Z, SP, false, DTPK>), dim3((unsigned)(ntiles * a.Bt * nseg)),
+                       dim3(512), 0, a.stream, pa, (const T*)a.u, (const T*)a.delta, (const T*)a.B,
+                       (const T*)a.C, (const T*)a.z, (T*)a.out);
+    HX_LAUNCH_CHECK();
+    return HX_OK;
+}
+template <typename T>
+int dispatch_ps(const ScanArgs& a) {
+    const bool hz = a.z != nullptr;
+    if (hz && a.softplus) return launch_ps<T, true, true, 0>(a, nullptr, nullptr);
+    if (hz) return launch_ps<T, true, false, 0>(a, nullptr, nullptr);
+    if (a.softplus) return launch_ps<T, false, true, 0>(a, nullptr, nullptr);
+    return launch_ps<T, false, false, 0>(a, nullptr, nullptr);
 }
 
 template <typename T, int W, int TCH, bool HAS_Z, bool SP>
@@ -1953,7 +2032,18 @@ int run_scan(const ScanArgs& a) {
                          aligned(a.out, 16) && (!a.z || aligned(a.z, 16)) &&
                          (!a.D || aligned(a.D, 16)) && (!a.dt_bias || aligned(a.dt_bias, 16)) &&
                          a.Bt * ((a.Dm + 63) / 64) <= 0x7fffffff;
-    if (v == 0) {  // auto: the wave-complete kernels where their float4 access is legal
+    if (v == 0) {
+        // auto: scan_ps_kernel; fp32 that fits one block per CU of the split-state warp-specialised
+        // kernel, whose 48-channel blocks spread such a size over a third more CUs than 64-channel
+        // ones (8 x 2048 x 1536: 128 us against 135), unless the sequence is cut; sizes past the paired kernel's
+        // offsets take the wave kernels where their float4 access is legal
+        if (ps_ok(a.Bt, a.Dm, a.L, es)) {
+            const bool cut = a.ws && ps_segments(a.Bt, a.Dm, a.L) > 1;
+            if constexpr (std::is_same<T, float>::value)
+                if (!cut && tile_ok && ws2_ok<T>(a) && a.Bt * ((a.Dm + 47) / 48) <= device_cus())
+                    return dispatch_ws<T, 3, true>(a);
+            return dispatch_ps<T>(a);
+        }
         if (tile_ok) {
             if (ws_preferred(a, sizeof(T))) {
                 // fp32: the split-state form (two waves per SIMD; config 2 132.5 vs 145.4 us).
@@ -1984,6 +2074,8 @@ int run_scan(const ScanArgs& a) {
 // a path that needs none leaves a given workspace unused).
 size_t scan_workspace_bytes(const ScanArgs& a, size_t es) {
     const int v = g_scan_variant;
+    if (a.N == 16 && v == 0 && a.L > 0 && a.Bt > 0 && a.Dm > 0 && ps_ok(a.Bt, a.Dm, a.L, es))
+        return ps_workspace_bytes(a.Bt, a.Dm, a.L);
     if (a.N != 16 || a.Dm % 4 != 0 || a.L <= 0 || a.Bt <= 0 || a.Dm <= 0) return 0;
     if (v != 0 && v != 40 && v != 42) return 0;  // generic, fast and warp-specialised: none
     if (v == 0 && ws_preferred(a, es)) return 0;
@@ -2039,6 +2131,19 @@ int scan_entry(int64_t batch, int64_t seqlen, int64_t dim, int64_t dstate, int d
 }  // namespace hx
 
 namespace hx {
+int scan_fwd_scratch(int64_t batch, int64_t seqlen, int64_t dim, const uint16_t* u, const uint16_t* delta,
+                     const float* A, const uint16_t* B, const uint16_t* C, const float* D, const uint16_t* z,
+                     const float* dt_bias, uint16_t* out, float* last_state, void* ws, size_t ws_bytes,
+                     hipStream_t stream) {
+    ScanArgs a{batch, seqlen, dim, 16, 1, u, delta, A, B, C, D, z, dt_bias, out, nullptr, last_state, stream};
+    if (g_scan_variant == 0 && g_scan_segments == 0 && ps_ok(batch, dim, seqlen, 2)) {
+        a.ws = ws;
+        a.ws_bytes = ws_bytes;
+        a.ws_may_be_short = true;
+    }
+    return run_scan<uint16_t>(a);
+}
+
 bool scan_variant_is_auto() { return g_scan_variant == 0; }
 
 bool scan_dtproj_ok(int64_t batch, int64_t seqlen, int64_t dim, int64_t rank) {
@@ -2049,7 +2154,7 @@ bool scan_dtproj_ok(int64_t batch, int64_t seqlen, int64_t dim, int64_t rank) {
 int scan_fwd_dtproj(int64_t batch, int64_t seqlen, int64_t dim, const uint16_t* u, const uint16_t* dtlo,
                     int64_t rank, const uint16_t* w_dt, const float* A, const uint16_t* B,
                     const uint16_t* C, const float* D, const uint16_t* z, const float* dt_bias,
-                    uint16_t* out, float* last_state, hipStream_t stream) {
+                    uint16_t* out, float* last_state, void* ws, size_t ws_bytes, hipStream_t stream) {
     HX_REQUIRE(scan_dtproj_ok(batch, seqlen, dim, rank), HX_ERR_UNSUPPORTED,
                "selective scan with dt_proj: sizes outside the fused path (batch %lld, seqlen %lld, "
                "dim %lld, dt_rank %lld)", (long long)batch, (long long)seqlen, (long long)dim, (long long)rank);
@@ -2060,6 +2165,16 @@ int scan_fwd_dtproj(int64_t batch, int64_t seqlen, int64_t dim, const uint16_t* 
     HX_REQUIRE(aligned(u, 16) && aligned(z, 16) && aligned(out, 16) && aligned(dtlo, 16) && aligned(w_dt, 16) &&
                    aligned(B, 32) && aligned(C, 32) && (!D || aligned(D, 16)) && (!dt_bias || aligned(dt_bias, 16)),
                HX_ERR_UNSUPPORTED, "selective scan with dt_proj: operands not 16-byte aligned");
+    if (ps_ok(batch, dim, seqlen, 2)) {
+        const ScanArgs a{batch, seqlen, dim, 16, 1, u, nullptr, A, B, C, D, z, dt_bias, out, nullptr, last_state,
+                         stream, ws, ws_bytes, true};
+        switch (rank / 32) {
+            case 1: return launch_ps<uint16_t, true, true, 1>(a, dtlo, w_dt);
+            case 2: return launch_ps<uint16_t, true, true, 2>(a, dtlo, w_dt);
+            case 3: return launch_ps<uint16_t, true, true, 3>(a, dtlo, w_dt);
+            default: return launch_ps<uint16_t, true, true, 4>(a, dtlo, w_dt);
+        }
+    }
     constexpr int WPB = 4;
     const int64_t ntiles = (dim + 16 * WPB - 1) / (16 * WPB);
     WaveSeg sg{seqlen, 1, nullptr, nullptr, nullptr};
@@ -2093,7 +2208,7 @@ extern "C" int hx_selective_scan_dtproj_fwd(int64_t batch, int64_t seqlen, int64
     if (batch == 0 || dim == 0) return HX_OK;
     return scan_fwd_dtproj(batch, seqlen, dim, (const uint16_t*)u, (const uint16_t*)dt_lo, dt_rank,
                            (const uint16_t*)w_dt, A, (const uint16_t*)B, (const uint16_t*)C, D,
-                           (const uint16_t*)z, dt_bias, (uint16_t*)out, last_state, as_stream(stream));
+                           (const uint16_t*)z, dt_bias, (uint16_t*)out, last_state, nullptr, 0, as_stream(stream));
 }
 
 extern "C" int hx_selective_scan_fwd(int64_t batch, int64_t seqlen, int64_t dim, int64_t dstate,

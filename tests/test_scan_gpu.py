@@ -403,3 +403,68 @@ def test_scan_dtproj_errors_and_empty(dev):
     call(args(64, seq=0), 64, seq=0, last=last)
     torch.cuda.synchronize()
     assert torch.equal(last, torch.zeros_like(last))
+
+
+@pytest.mark.parametrize("with_z", [True, False])
+@pytest.mark.parametrize("bt,L,dim", [(1, 1, 4), (2, 15, 68), (3, 16, 64), (2, 17, 60), (1, 47, 128), (2, 48, 192),
+                                      (2, 49, 132), (1, 97, 1000), (5, 250, 64)])
+def test_scan_paired_kernel_matches_wave_kernel_bitwise(dev, bt, L, dim, with_z):
+    """bf16's automatic kernel (state and element waves in pairs) performs the wave kernel's (42)
+    operations in its order: the same bits around its edges, 16-step chunks in rounds of three and
+    64-channel tiles, with an initial state and the final state."""
+    x = scan_inputs(bt, L, dim, 16, seed=L * 7 + dim, with_z=with_z, with_bias=True)
+    init = (np.random.default_rng(L).standard_normal((bt, dim, 16)) * 0.5).astype(np.float32)
+    ssm.set_scan_segments(1)
+    try:
+        auto = run_gpu(x, dev, dtype=torch.bfloat16, init_state=init, last=True)
+        ssm.set_scan_variant(42)
+        wave = run_gpu(x, dev, dtype=torch.bfloat16, init_state=init, last=True)
+    finally:
+        ssm.set_scan_segments(0)
+    assert np.array_equal(auto[0], wave[0])
+    assert np.array_equal(auto[1], wave[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("bt,L,dim", [(1, 512, 64), (1, 555, 5), (2, 1000, 70), (1, 4113, 33), (43, 600, 128),
+                                      (1, 2048, 1536)])
+def test_scan_automatic_segments(dev, bt, L, dim, dtype):
+    """Sizes whose tiles leave CUs idle are cut into time segments by themselves: at most half a round
+    of tiles, ragged last segments and chunks, dims outside the wave kernels' multiples of 4. Held to
+    the float64 restatement: outputs to their bar (fp32: or 1.5x the sequential f32 oracle's own
+    distance), the final state normwise: a step rounds it three times by at most 2^-24 of it, and
+    independent errors of L steps, undamped at worst, add up to sqrt(3 L) 2^-24, four sigma of it here."""
+    x = scan_inputs(bt, L, dim, 16, seed=L + dim, with_bias=True)
+    if dtype == torch.bfloat16:
+        x = {k: (bf16_round(v) if k not in ("A", "D", "dt_bias") else v) for k, v in x.items()}
+    init = (np.random.default_rng(L).standard_normal((bt, dim, 16)) * 0.5).astype(np.float32)
+    assert ssm.selective_scan_workspace_size(bt, L, dim, 16, dtype) > 0
+    g, glast = run_gpu(x, dev, dtype=dtype, init_state=init, last=True)
+    r = oracle.selective_scan(**x, init_state=init)
+    r64, rlast64 = oracle.numpy_selective_scan(**x, init_state=init)
+    assert norm_err(glast, rlast64) <= 4 * (3 * L) ** 0.5 * 2.0 ** -24
+    assert rel_err(g, r64) <= (TOL_BF16 if dtype == torch.bfloat16 else max(TOL_F32, 1.5 * rel_err(r, r64)))
+
+
+def test_scan_workspace_below_the_size_asked_for(dev):
+    """A kept workspace smaller than the size asked for: below 4096 steps the sequence is cut into the
+    segments that fit (one, with no whole segment's room), from there the call is refused."""
+    x = scan_inputs(1, 1000, 64, 16, seed=3)
+    r64, _ = oracle.numpy_selective_scan(**x)
+    need = ssm.selective_scan_workspace_size(1, 1000, 64, 16)
+    from helixml_amd import _ffi
+    d = {k: to_dev(v, dev) for k, v in x.items()}
+    for nbytes in (16, need // 2, need):
+        out = torch.full_like(d["u"], float("nan"))
+        ws = torch.empty(need, device=dev, dtype=torch.uint8)
+        _ffi.call("hx_selective_scan_fwd_ws", 1, 1000, 64, 16, _ffi.HX_F32, 1,
+                  *[d[k].data_ptr() if d[k] is not None else None for k in ("u", "delta", "A", "B", "C", "D", "z", "dt_bias")],
+                  out.data_ptr(), None, None, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert rel_err(out.cpu().numpy(), r64) <= TOL_F32, nbytes
+    z = torch.zeros(1, 8192, 64, device=dev)
+    bc = torch.zeros(1, 8192, 16, device=dev)
+    with pytest.raises(InvalidInput):
+        _ffi.call("hx_selective_scan_fwd_ws", 1, 8192, 64, 16, _ffi.HX_F32, 1, z.data_ptr(), z.data_ptr(),
+                  d["A"].data_ptr(), bc.data_ptr(), bc.data_ptr(), None, None, None, z.data_ptr(), None, None,
+                  ws.data_ptr(), 16, torch.cuda.current_stream().cuda_stream)
