@@ -217,6 +217,103 @@ __global__ __launch_bounds__(256) void s4_input_proj_kernel(int64_t M, int64_t L
     }
 }
 
+// The same sums for sequences too short to fill the chip with the blocks above: a block of 4 waves owns
+// 64 steps (lane = step) and 4 states, one a wave, so a row of x costs a wave one chain's product and sum
+// instead of eight. Rows go straight to a 4-slot LDS ring of 64 rows, three slots ahead (every wave
+// loads a quarter of them); dt * B[n][m], rounded as the reference rounds it, is formed in LDS without a
+// launch before this one (uniform loads of B, each a miss of the scalar cache, took 18 us). Bound by the chain's issue and
+// the LDS reads' latency, about 20 cycles a row. 512 x 256, 16 states: 43 us on the two blocks of the
+// kernel above and 19 with one wave a block whose rows came through registers, 16 here.
+constexpr int kPlRows = 64, kPlSlots = 4;
+constexpr int kPlMaxM = 2048;  // Bd rows: 4 x 8 KB of LDS beside the ring's 64 KB
+// v[k] = the float at LDS byte offset a + (R0 + k) * 256 and b[k] = the float at offset ab + 4 k, k < 16;
+// complete inside the statement, as lds_rows4
+template <int R0>
+__device__ inline void lds_rows16(uint32_t a, uint32_t ab, float (&v)[16], float (&b)[16]) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    hx_f32x2 r0, r1, r2, r3, r4, r5, r6, r7;
+    f32x4 b0, b1, b2, b3;
+    asm volatile(
+        "ds_read2st64_b32 %0, %12 offset0:%14 offset1:%14+1\n\t"
+        "ds_read_b128 %8, %13\n\t"
+        "ds_read2st64_b32 %1, %12 offset0:%14+2 offset1:%14+3\n\t"
+        "ds_read2st64_b32 %2, %12 offset0:%14+4 offset1:%14+5\n\t"
+        "ds_read_b128 %9, %13 offset:16\n\t"
+        "ds_read2st64_b32 %3, %12 offset0:%14+6 offset1:%14+7\n\t"
+        "ds_read2st64_b32 %4, %12 offset0:%14+8 offset1:%14+9\n\t"
+        "ds_read_b128 %10, %13 offset:32\n\t"
+        "ds_read2st64_b32 %5, %12 offset0:%14+10 offset1:%14+11\n\t"
+        "ds_read2st64_b32 %6, %12 offset0:%14+12 offset1:%14+13\n\t"
+        "ds_read_b128 %11, %13 offset:48\n\t"
+        "ds_read2st64_b32 %7, %12 offset0:%14+14 offset1:%14+15\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(r0), "=&v"(r1), "=&v"(r2), "=&v"(r3), "=&v"(r4), "=&v"(r5), "=&v"(r6), "=&v"(r7), "=&v"(b0),
+          "=&v"(b1), "=&v"(b2), "=&v"(b3)
+        : "v"(a), "v"(ab), "n"(R0)
+        : "memory");
+    const hx_f32x2 r[8] = {r0, r1, r2, r3, r4, r5, r6, r7};
+    const f32x4 q[4] = {b0, b1, b2, b3};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) { v[2 * k] = r[k][0]; v[2 * k + 1] = r[k][1]; }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) b[k] = q[k / 4][k % 4];
+}
+__global__ __launch_bounds__(256) void s4_proj_lane_kernel(int64_t M, int64_t L, int64_t N, float dt,
+                                                           const float* __restrict__ x,
+                                                           const float* __restrict__ B, float* __restrict__ U) {
+#pragma clang fp contract(off)
+    __shared__ __attribute__((aligned(16))) float ring[kPlSlots][kPlRows][64];
+    extern __shared__ __attribute__((aligned(16))) float s_bd[];  // [4][M rounded up to 16 rows]
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t t = (int64_t)blockIdx.x * 64 + lane;
+    const int64_t n = (int64_t)blockIdx.y * 4 + w, nc = n < N ? n : N - 1;
+    const float* xt = x + (t < L ? t : L - 1);
+    constexpr int P = kPlRows / 4, WAITN = P * (kPlSlots - 2);
+    static_assert(WAITN <= 63, "vmcnt range");
+    // wave w loads rows 4 i + w of every chunk; rows past M read row M - 1 (every chunk the same count)
+    auto issue = [&](int64_t q) __attribute__((always_inline)) {
+        float(*dst)[64] = ring[q % kPlSlots];
+        const int64_t m0 = q * kPlRows + w;
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            const int64_t m = m0 + 4 * i < M ? m0 + 4 * i : M - 1;
+            __builtin_amdgcn_global_load_lds((gvoid_t*)(xt + m * L), (lvoid_t*)&dst[4 * i + w][0], 4, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < kPlSlots - 1; ++q) issue(q);
+    const int64_t nch = (M + kPlRows - 1) / kPlRows;
+    const uint32_t base = lds_off(&ring[0][0][lane]);
+    float acc = 0.0f;
+    float* bd = s_bd + w * ((M + 15) / 16 * 16);
+    for (int64_t m = lane; m < M; m += 64) bd[m] = __fmul_rn(B[nc * M + m], dt);
+    const uint32_t bbase = lds_off(bd);
+    for (int64_t c = 0; c < nch; ++c) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAITN) : "memory");     // own loads of chunk c
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // everyone's; chunk c - 1 is read
+        issue(c + kPlSlots - 1);
+        const uint32_t ca = base + (uint32_t)(c % kPlSlots) * (kPlRows * 256);
+        StepLoop<kPlRows / 16>::run([&](auto gc) __attribute__((always_inline)) {
+            constexpr int g = decltype(gc)::value;
+            const int64_t m0 = c * kPlRows + 16 * g;
+            if (m0 + 16 <= M) {
+                float xv[16], bq[16];
+                lds_rows16<16 * g>(ca, bbase + (uint32_t)m0 * 4, xv, bq);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc = __fadd_rn(acc, __fmul_rn(bq[i], xv[i]));
+            } else {
+                for (int64_t m = m0; m < M; ++m) {
+                    const float xv = lds_row1(ca + (uint32_t)(m - c * kPlRows) * 256);
+                    acc = __fadd_rn(acc, __fmul_rn(lds_row1(bbase + (uint32_t)m * 4), xv));
+                }
+            }
+        });
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load still writing LDS at exit
+    if (t < L && n < N) U[t * N + n] = acc;
+}
+
 // BdT[m][n] = B[n][m] * dt for n < N, 0 for N <= n < Np (mul_scalar, ssm.rs:130), rounded once
 // like the reference; transposed and padded for the projection's scalar loads.
 __global__ void s4_scale_kernel(int64_t M, int64_t N, int64_t Np, float dt,
@@ -421,6 +518,85 @@ __global__ __launch_bounds__(256) void s4_output_kernel(int64_t M, int64_t L, in
         float v = __fadd_rn(o, __fmul_rn(dd, sx[mm][tt]));
         if (gate) v = __fmul_rn(v, g);
         y[t * M + m] = v;
+    }
+}
+
+// Recurrence and output in one launch for short sequences (N <= 16, L <= kFuseT): a block copies the
+// projection's U for every step up to its tile's end to LDS, one wave runs the chains over it (in
+// place, s1 = a*h then + U, each rounded; about 20 cycles a step) and the tile's outputs follow as in
+// s4_output_kernel. Every block repeats the chain from step 0, which up to kFuseT steps costs less than
+// the launch and the round trip through memory that it saves (512 x 256: 13 us against 8 + 5 and a gap before each).
+constexpr int kFuseT = 512, kFuseTile = 16;
+__global__ __launch_bounds__(256) void s4_scan_output_kernel(int64_t M, int64_t L, int N,
+                                                             const float* __restrict__ x,
+                                                             const float* __restrict__ a,
+                                                             const float* __restrict__ U,
+                                                             const float* __restrict__ C,
+                                                             const float* __restrict__ D,
+                                                             const float* __restrict__ gate,
+                                                             float* __restrict__ y) {
+#pragma clang fp contract(off)
+    __shared__ float sx[kTileM][kFuseTile + 1];
+    __shared__ float sh[kFuseT + 32][16];  // the chain reads ahead
+    const int64_t m0 = (int64_t)blockIdx.x * kTileM;
+    const int t0 = (int)blockIdx.y * kFuseTile;
+    const int t1 = t0 + kFuseTile < (int)L ? t0 + kFuseTile : (int)L;
+    const int tid = threadIdx.x;
+    {
+        const int n = tid & 15;
+#pragma unroll 8
+        for (int t = tid >> 4; t < t1; t += 16) sh[t][n] = n < N ? U[t * N + n] : 0.0f;
+    }
+    for (int i = tid; i < kTileM * kFuseTile; i += 256) {
+        const int mm = i / kFuseTile, tt = i % kFuseTile;
+        const int64_t m = m0 + mm;
+        sx[mm][tt] = (m < M && t0 + tt < L) ? x[m * L + t0 + tt] : 0.0f;
+    }
+    const int mm = tid & 63;
+    const int64_t m = m0 + mm, mc = m < M ? m : M - 1;
+    float c[16];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) c[n] = n < N ? C[mc * N + n] : 0.0f;
+    const float dd = D[mc];
+    const float g = gate ? gate[mc] : 1.0f;
+    __syncthreads();
+    if (tid < N) {
+        const float an = a[tid];
+        float h = 0.0f, va[16], vb[16];
+        auto read = [&](float (&v)[16], int t) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < 16; ++k) v[k] = sh[t + k][tid];
+        };
+        // 16 steps whose U was read 16 steps ahead; steps past t1 run on unused values
+        auto chain = [&](float (&v)[16], int t) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                h = __fadd_rn(__fmul_rn(an, h), v[k]);
+                v[k] = h;
+            }
+            if (t + 16 > t0)
+#pragma unroll
+                for (int k = 0; k < 16; ++k) sh[t + k][tid] = v[k];
+        };
+        read(va, 0);
+        for (int t = 0; t < t1; t += 32) {
+            read(vb, t + 16);
+            chain(va, t);
+            if (t + 16 >= t1) break;
+            read(va, t + 32 <= kFuseT ? t + 32 : kFuseT);
+            chain(vb, t + 16);
+        }
+    }
+    __syncthreads();
+    if (m >= M) return;
+    for (int t = t0 + (tid >> 6); t < t1; t += 4) {
+        float o = 0.0f;
+#pragma unroll
+        for (int n = 0; n < 16; ++n)
+            if (n < N) o = __fadd_rn(o, __fmul_rn(c[n], sh[t][n]));
+        float v = __fadd_rn(o, __fmul_rn(dd, sx[mm][t - t0]));
+        if (gate) v = __fmul_rn(v, g);
+        y[(int64_t)t * M + m] = v;
     }
 }
 
@@ -1051,6 +1227,18 @@ extern "C" int hx_s4_discretize(int64_t dstate, float dt, const float* a_real, c
     return HX_OK;
 }
 
+namespace hx {
+namespace {
+// Whether s4_proj_lane_kernel takes the bit-exact projection: up to one of its waves per SIMD (whole
+// calls, 16 states: 2048 x 4096 113 us against 222 with the ring kernel, 512 x 4096 66 against 93; with
+// four waves it is behind, 2048 x 16384 432 against 365), Bd rows that fit beside the ring in LDS.
+bool s4_proj_lane_ok(int64_t M, int64_t N, int64_t L) {
+    return M <= kPlMaxM && (L + 63) / 64 * N <= 1024 &&
+           grant_dynamic_lds((const void*)s4_proj_lane_kernel, (size_t)kPlMaxM * 16, (size_t)kPlSlots * kPlRows * 256);
+}
+}  // namespace
+}  // namespace hx
+
 extern "C" size_t hx_s4_ref_workspace_size(int64_t d_model, int64_t dstate, int64_t seqlen) {
     if (d_model <= 0 || dstate <= 0 || seqlen <= 0) return 0;
     return hx::s4_ref_ws_bytes(d_model, dstate, seqlen);
@@ -1080,15 +1268,27 @@ extern "C" int hx_s4_ref_fwd(int64_t d_model, int64_t dstate, int64_t seqlen, fl
     float* BdT = (float*)workspace;
     float* H = (float*)((char*)workspace + align256((size_t)Np * d_model * sizeof(float)));
     const size_t n_bd = (size_t)Np * d_model;
-    hipLaunchKernelGGL(s4_scale_kernel, dim3((unsigned)((n_bd + 255) / 256)), dim3(256), 0, s,
-                       d_model, dstate, Np, dt, B, BdT);
-    const dim3 g1((unsigned)((seqlen + kPjT - 1) / kPjT), (unsigned)(Np / 8));
-    if (seqlen % 4 == 0 && aligned(x, 16))
-        hipLaunchKernelGGL(s4_input_proj_kernel<16>, g1, dim3(256), 0, s, d_model, seqlen, dstate,
-                           Np, x, BdT, H);
-    else
-        hipLaunchKernelGGL(s4_input_proj_kernel<4>, g1, dim3(256), 0, s, d_model, seqlen, dstate,
-                           Np, x, BdT, H);
+    if (s4_proj_lane_ok(d_model, dstate, seqlen)) {
+        hipLaunchKernelGGL(s4_proj_lane_kernel, dim3((unsigned)((seqlen + 63) / 64), (unsigned)((dstate + 3) / 4)),
+                           dim3(256), (size_t)(d_model + 15) / 16 * 256, s, d_model, seqlen, dstate, dt, x, B, H);
+    } else {
+        hipLaunchKernelGGL(s4_scale_kernel, dim3((unsigned)((n_bd + 255) / 256)), dim3(256), 0, s,
+                           d_model, dstate, Np, dt, B, BdT);
+        const dim3 g1((unsigned)((seqlen + kPjT - 1) / kPjT), (unsigned)(Np / 8));
+        if (seqlen % 4 == 0 && aligned(x, 16))
+            hipLaunchKernelGGL(s4_input_proj_kernel<16>, g1, dim3(256), 0, s, d_model, seqlen, dstate,
+                               Np, x, BdT, H);
+        else
+            hipLaunchKernelGGL(s4_input_proj_kernel<4>, g1, dim3(256), 0, s, d_model, seqlen, dstate,
+                               Np, x, BdT, H);
+    }
+    if (dstate <= 16 && seqlen <= kFuseT) {
+        hipLaunchKernelGGL(s4_scan_output_kernel, dim3((unsigned)((d_model + kTileM - 1) / kTileM),
+                                                       (unsigned)((seqlen + kFuseTile - 1) / kFuseTile)),
+                           dim3(256), 0, s, d_model, seqlen, (int)dstate, x, a, H, C, D, gate, y);
+        HX_LAUNCH_CHECK();
+        return HX_OK;
+    }
     const bool pow2 = (dstate & (dstate - 1)) == 0;
     if (pow2 && (seqlen * dstate) % 4 == 0) {
         int lgN = 0;
