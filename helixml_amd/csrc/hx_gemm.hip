@@ -731,14 +731,15 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_dlds_kernel(int64_t M, int64
 // ----------------------------------------------------------------------------- narrow N
 // Products with few output columns and a long K (the block's x_proj: N = dt_rank + 2 dstate, 160
 // at config 3 and 64 at config 5, K = d_inner), which stream X from HBM once: a block owns 64 rows
-// and every column, so the grid is M / 64 blocks and no K split is needed. Block tile 64 x NB
+// and every column, so the grid is M / 64 blocks and no K split is needed. (Products of middle size
+// run it over a second grid axis of column tiles, CB = 1 or 2.) Block tile 64 x NB
 // (NB = 64 CB, N <= NB): 4 waves in 2 x 2, each 32 rows x 32 CB columns (CB
 // v_mfma_f32_32x32x16_bf16 per 16-wide K step, K ascending as in the other kernels, so each
 // output is the same sum). K tiles of 64 move straight into a 3- or 4-stage LDS ring with
 // global_load_lds_dwordx4 (A rows 0..63, then W rows 0..NB-1, 128-byte rows with the 16-byte
 // chunks XOR-swizzled by row); the loads of tile kt+2 (kt+3) are issued while tile kt is multiplied.
-// W (at most NB x K) is read by every block and stays in L2. Requires K % 64 == 0 and 16-byte
-// aligned rows; rows past M or N are clamped (their outputs are discarded).
+// W (at most NB x K) is read by every block and stays in L2. Requires K % 8 == 0 and 16-byte
+// aligned rows; a last K tile past K reads zeros; rows past M or N are clamped (their outputs are discarded).
 constexpr int NBM = 64;
 
 template <int CB>
@@ -749,6 +750,9 @@ constexpr int narrow_stage_bytes() { return (NBM + 64 * CB) * 128; }
 // CB = 1, 50.8 -> 54.3 us with 4).
 template <int CB>
 constexpr int narrow_stages() { return CB >= 3 ? 4 : 3; }
+
+// What the lanes of a ragged last K tile read past K.
+__device__ const uint16_t kZeros[8] = {};
 
 template <int CB>
 __global__ __launch_bounds__(256) void gemm_bf16_nt_narrow_kernel(int64_t M, int64_t N, int64_t K,
@@ -768,6 +772,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_narrow_kernel(int64_t M, int
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int64_t m0 = (int64_t)blockIdx.x * NBM;
+    const int64_t n0 = (int64_t)blockIdx.y * (64 * CB);
 
     // region q = QW * wave + j of a stage: rows 8q .. 8q + 7 (0..63 = A, then W); lane L fills
     // row 8q + L / 8, slot L % 8 with K-chunk (L % 8) ^ (row & 7)
@@ -781,16 +786,23 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_narrow_kernel(int64_t M, int
             const int64_t gr = m0 + row < M ? m0 + row : M - 1;
             src[j] = X + gr * ldx + chunk * 8;
         } else {
-            const int64_t gr = row - NBM < N ? row - NBM : N - 1;
+            const int64_t gr = n0 + row - NBM < N ? n0 + row - NBM : N - 1;
             src[j] = W + gr * ldw + chunk * 8;
         }
     }
     auto issue = [&](int64_t kt) __attribute__((always_inline)) {
         char* stage = sbase + (int)(kt % NST3) * SB;
+        const uint16_t* p[QW];
+#pragma unroll
+        for (int j = 0; j < QW; ++j) p[j] = src[j] + kt * 64;
+        if (kt * 64 + 64 > K) {  // a last tile past K: its pieces (K % 8 == 0: whole ones) read zeros
+#pragma unroll
+            for (int j = 0; j < QW; ++j)
+                if (kt * 64 + 8 * ((lane & 7) ^ (lane >> 3)) >= K) p[j] = kZeros;
+        }
 #pragma unroll
         for (int j = 0; j < QW; ++j)
-            __builtin_amdgcn_global_load_lds((gvoid_t*)(src[j] + kt * 64),
-                                             (lvoid_t*)(stage + (wave * QW + j) * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gvoid_t*)p[j], (lvoid_t*)(stage + (wave * QW + j) * 1024), 16, 0, 0);
     };
 
     f32x16 acc[CB];
@@ -801,7 +813,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_narrow_kernel(int64_t M, int
 
     const int fr = lane & 31;
     const int fc = lane >> 5;
-    const int64_t nk = K / 64;
+    const int64_t nk = (K + 63) / 64;
 #pragma unroll
     for (int t = 0; t < NST3 - 1; ++t)
         if (t < nk) issue(t);
@@ -843,7 +855,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_narrow_kernel(int64_t M, int
     // 32 x 64 slabs staged per wave (two column blocks at a time); the wave's columns end at
     // n_end, past which a slab's second half (odd CB) holds no result
     float* st = reinterpret_cast<float*>(smem) + wave * (32 * 68);
-    const int64_t c0 = (int64_t)wn * 32 * CB;
+    const int64_t c0 = n0 + (int64_t)wn * 32 * CB;
     const int64_t n_end = c0 + 32 * CB < N ? c0 + 32 * CB : N;
 #pragma unroll
     for (int g = 0; g < (CB + 1) / 2; ++g) {
@@ -1509,7 +1521,8 @@ int launch_narrow_cb(int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx
                "gemm_bf16: the device does not grant %zu bytes of LDS", bytes);
     HX_REQUIRE((M + NBM - 1) / NBM <= 0x7fffffff, HX_ERR_UNSUPPORTED, "gemm_bf16: M=%lld too large",
                (long long)M);
-    hipLaunchKernelGGL((gemm_bf16_nt_narrow_kernel<CB>), dim3((unsigned)((M + NBM - 1) / NBM)), dim3(256),
+    hipLaunchKernelGGL((gemm_bf16_nt_narrow_kernel<CB>),
+                       dim3((unsigned)((M + NBM - 1) / NBM), (unsigned)((N + 64 * CB - 1) / (64 * CB))), dim3(256),
                        bytes, as_stream(stream), M, N, K, (const uint16_t*)X, ldx, (const uint16_t*)W, ldw,
                        bias, o);
     HX_LAUNCH_CHECK();
@@ -1651,16 +1664,25 @@ extern "C" int hx_gemm_bf16(int64_t M, int64_t N, int64_t K, const void* X, int6
         return launch_d256<64, 2>(M, N, K, X, ldx, W, ldw, bias, o, stream);
     if (vec && K > 0 && K % 32 == 0 && (g_gemm_kernel == 6 || (d256_auto && K % 64 != 0)) && d256_ok<32, 4>())
         return launch_d256<32, 4>(M, N, K, X, ldx, W, ldw, bias, o, stream);
+    // auto, too few 256 x 256 tiles for one per CU. From 112 of them that kernel still leads (4000 x 2048 x
+    // 512: 20 us against 26 with 64 x 128 tiles; at 96, 1999 x 3072 x 768, 31 against 26). Below, and where K
+    // is no multiple of 64, the narrow kernel's 64-row tiles over a grid of columns: 128 wide, or 64 where
+    // those leave CUs idle (777 x 1024 x 2048, 104 wide tiles: 18 us against 21). Against the kernels
+    // that took these before: 1999 x 768 x 1536 38 -> 18 us, 2867 x 1736 x 3472 133 -> 84, 48 x 2048 x 4096
+    // 76 -> 26. Same K-ascending 16-wide MFMA sums as the 256 x 256 kernel's, so a short batch that
+    // lands here matches a long one there. Short K and few outputs stay with the small-M kernel (1000 x
+    // 512 x 1024: 8.5 us against 10.5; level at 32-square tiles x K of 2^19: 500 x 2048 x 512), except from
+    // K = 2048 on, where its K split would give a prefix other bits than the whole.
+    const bool small_out = K < 2048 && ((M + 31) / 32) * ((N + 31) / 32) * K <= (1 << 19);
+    if (g_gemm_kernel == 0 && vec && K % 8 == 0 && K >= 64 && !small_out) {
+        if (K % 64 == 0 && N >= 256 && M >= 256 && ((M + XBM - 1) / XBM) * ((N + XBN - 1) / XBN) >= 112 && d256_ok<64, 2>())
+            return launch_d256<64, 2>(M, N, K, X, ldx, W, ldw, bias, o, stream);
+        if ((N + 63) / 64 <= 65535)
+            return ((M + 63) / 64) * ((N + 127) / 128) < 160 ? launch_narrow_cb<1>(M, N, K, X, ldx, W, ldw, bias, o, stream)
+                                                             : launch_narrow_cb<2>(M, N, K, X, ldx, W, ldw, bias, o, stream);
+    }
     const size_t dlds = (size_t)DSTAGES * DSTAGE_BYTES;
-    // auto: the direct-to-LDS kernel for long K (measured ahead of the 128 x 128 kernel from
-    // K = 2048 on, and from K = 1024 for N <= 128 where its tiles fill half the GPU: config 5
-    // x_proj 78 vs 87 us; behind it at K <= 512 where its one block per CU cannot hide the
-    // epilogue). Its per-element arithmetic is the 256 x 256 kernel's (K ascending in 16-wide
-    // MFMA steps), so a short batch that lands here matches a long one that takes that kernel.
-    const int64_t tiles_dlds = ((M + LBM - 1) / LBM) * ((N + LBN - 1) / LBN);
-    if (vec && K > 0 && K % LBK == 0 &&
-        (g_gemm_kernel == 4 ||
-         (g_gemm_kernel == 0 && (K >= 2048 || (K >= 1024 && N <= 128 && tiles_dlds >= 128)))) &&
+    if (vec && K > 0 && K % LBK == 0 && g_gemm_kernel == 4 &&
         dlds_ok(dlds)) {
         dim3 lg((unsigned)((N + LBN - 1) / LBN), (unsigned)((M + LBM - 1) / LBM));
         hipLaunchKernelGGL(gemm_bf16_nt_dlds_kernel, lg, dim3(256), dlds, as_stream(stream), M, N, K,
@@ -1670,7 +1692,7 @@ extern "C" int hx_gemm_bf16(int64_t M, int64_t N, int64_t K, const void* X, int6
     }
     const int64_t tiles128 = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     if (vec && K % 8 == 0 && K >= 8 && g_gemm_kernel != 1 && g_gemm_kernel != 4 &&
-        (g_gemm_kernel == 3 || tiles128 < 128) && (M + 31) / 32 <= 65535) {
+        (g_gemm_kernel == 3 || tiles128 < 128 || (g_gemm_kernel == 0 && small_out)) && (M + 31) / 32 <= 65535) {
         // 64-wide tiles where they still give the GPU 256 blocks (decode in_proj), else 32-wide;
         // SP covers a wave's whole share of K where it can (one round of loads). Where the grid
         // has at most one block per CU, blocks of 8 waves: each wave loads half the share, and two

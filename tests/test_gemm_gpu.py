@@ -357,3 +357,38 @@ def test_gemm_pointer_loads_past_2gib(dev, kernel):
     assert torch.equal(Y[M - 256:], tail)
     assert norm_err(tail.cpu().numpy(), ref(X[M - 256:], W)) <= 1e-5
     del X, Y
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (300, 264, 2056), (65, 129, 4096), (63, 64, 2048),     # 64-wide column tiles, a ragged last K tile
+    (1999, 768, 1544), (1100, 1000, 1096), (64, 33000, 72),  # 128-wide
+    (1792, 4096, 640), (1791, 4000, 640),                  # 112 tiles of 256 x 256 and their ragged form
+    (96, 4096, 1360), (96, 4104, 1360), (33, 40, 56),      # either side of the small-M kernel's 2^19
+])
+def test_gemm_middle_sizes(dev, M, N, K):
+    """The automatic choice between one tile of 256 x 256 per CU and the small-M kernel, at its edges:
+    fp32 outputs over three column splits, accumulated into what is there, and 16-bit outputs with bias
+    and SiLU. Products of bf16 values are exact in fp32, so an output is within K roundings of its
+    running sums, K 2^-24 of the summed magnitudes (and the bf16 rounding, 2^-8 of the result)."""
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    X = torch.randn(M, K, generator=g, device=dev).bfloat16()
+    W = (torch.randn(N, K, generator=g, device=dev) / K ** 0.5).bfloat16()
+    bias = torch.randn(N, generator=g, device=dev)
+    ref = X.double() @ W.double().T
+    bound = (K + 2) * 2.0 ** -24 * (X.double().abs() @ W.double().abs().T)
+    s1, s2 = N // 3, N // 3 + 8
+    outs = ssm.gemm_bf16(X, W, splits=(s1, s2), out_dtype=torch.float32)
+    y = torch.cat(outs, 1).double()
+    assert bool(((y - ref).abs() <= bound).all()), float((y - ref).abs().max())
+    yb = ssm.gemm_bf16(X, W, bias=bias, act=1).double()
+    v = ref + bias.double()
+    want = v * torch.sigmoid(v)
+    err = (yb - want).abs() - 2.0 ** -8 * want.abs() - 1.2 * bound - 1e-5
+    assert bool((err <= 0).all()), float(err.max())
+    if K % 64 == 0:  # the same sums as the 256 x 256 kernel's
+        ssm.set_gemm_kernel(5)
+        try:
+            same = ssm.gemm_bf16(X, W, out_dtype=torch.float32)
+        finally:
+            ssm.set_gemm_kernel(0)
+        assert torch.equal(same, torch.cat(outs, 1))
