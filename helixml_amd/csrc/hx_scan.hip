@@ -1791,6 +1791,10 @@ size_t ps_seg_bytes(int64_t Bt, int64_t Dm, int64_t nseg) {
 size_t ps_workspace_bytes(int64_t Bt, int64_t Dm, int64_t L) {
     return ps_seg_bytes(Bt, Dm, ps_seg_count(L, ps_seg_len(L, ps_segments(Bt, Dm, L))));
 }
+// Sequences given with a workspace may leave out what has decayed below kDecayDrop from this length on:
+// at dt near 0.02 the end-state pass of 65536 steps then walks about 1100 of each segment's 4096.
+// Shorter segments hardly reach that decay.
+constexpr int64_t kDropSteps = 4096;
 // scan_ps_kernel's sizes: a segment's byte offsets, a few chunks of read-ahead included, below 2^31.
 bool ps_ok(int64_t Bt, int64_t Dm, int64_t L, size_t es) {
     return L < (1LL << 30) && (L + 96) * Dm * (int64_t)es < (1LL << 31) && Bt * ((Dm + 63) / 64) <= 0x7fffffff;
@@ -1817,7 +1821,8 @@ int launch_ps(const ScanArgs& a, const uint16_t* dtlo, const uint16_t* wdt) {
                "selective scan: %lld blocks exceed the grid", (long long)(ntiles * a.Bt * nseg));
     float4* hend = (float4*)a.ws;
     float4* decay = hend + (nseg - 1) * a.Bt * ntiles * 256;
-    const PsArgs pa{a.L, a.Dm, (int)ntiles, (int)a.Bt, (int)nseg, (int)seg_len, a.A, a.D, a.dt_bias,
+    const PsArgs pa{a.L, a.Dm, (int)ntiles, (int)a.Bt, (int)nseg, (int)seg_len,
+                    a.L >= kDropSteps && !a.ws_may_be_short, a.A, a.D, a.dt_bias,
                     a.init_state, a.last_state, hend, decay, dtlo, wdt};
     if (nseg > 1) {
         hipLaunchKernelGGL((scan_ps_kernel<T, false, SP, true, DTPK>), dim3((unsigned)(ntiles * a.Bt * (nseg - 1))),

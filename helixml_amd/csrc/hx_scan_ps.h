@@ -12,6 +12,7 @@ struct PsArgs {
     int64_t L, Dm;
     int ntiles, Bt, nseg;
     int seg_len;                 // a multiple of 16; the last segment may be shorter
+    int drop;                    // END_ONLY: stop at kDecayDrop
     const float *A, *D, *bias, *init;
     float* last;
     float4 *hend, *decay;        // [nseg - 1][Bt][ntiles][4][64], nseg > 1
@@ -71,7 +72,10 @@ __device__ inline float to_f32(uint16_t v) { return bf16_bits_to_f32(v); }
 // it walks backwards from the end, adding exp2(A * S) * B*dt*u with S the sum of dt from there to the
 // end, and stops at the first 48-step round at which every state of the block's channels has decayed
 // below 2^-32 (kDecayDrop): what is left out is 2^-8 of the fp32 rounding of the state there. Such a
-// segment publishes decay 0. The output pass chains the segments before its own itself.
+// segment publishes decay 0. Below 4096 steps and in the Mamba block (drop = 0) it walks its whole
+// segment instead: a NaN, an infinity or an outlier reaches everything after it, as in the uncut scan,
+// and segments of a few hundred steps hardly ever decay that far. The output pass chains the segments
+// before its own itself.
 // Sizes: byte offsets inside a segment below 2^31.
 template <typename T, bool HAS_Z, bool SOFTPLUS, bool END_ONLY, int DTPK>
 __global__ __launch_bounds__(512, 4) void scan_ps_kernel(
@@ -136,7 +140,7 @@ __global__ __launch_bounds__(512, 4) void scan_ps_kernel(
         for (; i + NB <= nch; i += NB) {
             StepLoop<NB>::run([&](auto kc) __attribute__((always_inline)) { body(kc, i + decltype(kc)::value); });
             if constexpr (END_ONLY) {
-                if (stop_vote()) {
+                if (a.drop && stop_vote()) {
                     stopped(i + NB);
                     return 0;
                 }

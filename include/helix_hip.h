@@ -102,11 +102,12 @@ int hx_selective_scan_fwd(int64_t batch, int64_t seqlen, int64_t dim, int64_t ds
 /* hx_selective_scan_fwd with a caller workspace for cutting the sequence: when the (batch, channel)
  * tiles alone cannot fill the GPU (few channels and at least some hundred steps), the sequence is
  * cut into time segments whose end states (from a zero state) are accumulated backwards from
- * each segment's end until every state's decay to the end is below 2^-32, and every segment is then
- * scanned with outputs from the chained entry state (results agree with the unsegmented
- * scan to fp32 rounding). workspace: device memory of at least hx_selective_scan_workspace_size(...) bytes,
- * 16-byte aligned (0 bytes: no segments; fewer: as many segments as fit below 4096 steps, refused
- * from there); it holds no state between calls. Same reference
+ * each segment's end (from 4096 steps on until every state's decay to the end is below 2^-32, which
+ * leaves out what came before), and every segment is then scanned with outputs from the chained
+ * entry state (results agree with the unsegmented scan to fp32 rounding). workspace: device memory
+ * of at least hx_selective_scan_workspace_size(...) bytes, 16-byte aligned (0 bytes: no segments;
+ * fewer: below 4096 steps as many segments as fit, from there the call is refused); it holds no
+ * state between calls. Same reference
  * counterpart as hx_selective_scan_fwd (the per-step loop of ssm.rs:166-182). */
 size_t hx_selective_scan_workspace_size(int64_t batch, int64_t seqlen, int64_t dim,
                                         int64_t dstate, int dtype);

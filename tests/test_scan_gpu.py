@@ -468,3 +468,18 @@ def test_scan_workspace_below_the_size_asked_for(dev):
         _ffi.call("hx_selective_scan_fwd_ws", 1, 8192, 64, 16, _ffi.HX_F32, 1, z.data_ptr(), z.data_ptr(),
                   d["A"].data_ptr(), bc.data_ptr(), bc.data_ptr(), None, None, None, z.data_ptr(), None, None,
                   ws.data_ptr(), 16, torch.cuda.current_stream().cuda_stream)
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_scan_automatic_segments_keep_non_finite_values(dev, value):
+    """A sequence below 4096 steps that is cut by itself loses no NaN or infinity: one input early in the
+    first segment, with steps so large that its state decays by 2^-1000 before that segment ends, leaves
+    that channel's later outputs without a finite value, as the recurrence does, and no other channel's."""
+    x = scan_inputs(1, 1000, 64, 16, seed=5)
+    x["u"][0, 2, 7] = value
+    x["delta"][:] = 1.0
+    assert ssm.selective_scan_workspace_size(1, 1000, 64, 16) > 0
+    out, last = run_gpu(x, dev, last=True)
+    assert not np.isfinite(out[0, 2:, 7]).any() and not np.isfinite(last[0, 7]).any()
+    other = np.arange(64) != 7
+    assert np.isfinite(out[0][:, other]).all() and np.isfinite(out[0, :2, 7]).all()
