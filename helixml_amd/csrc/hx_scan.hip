@@ -1791,6 +1791,7 @@ size_t ps_seg_bytes(int64_t Bt, int64_t Dm, int64_t nseg) {
 size_t ps_workspace_bytes(int64_t Bt, int64_t Dm, int64_t L) {
     return ps_seg_bytes(Bt, Dm, ps_seg_count(L, ps_seg_len(L, ps_segments(Bt, Dm, L))));
 }
+size_t wave_workspace_bytes(const ScanArgs& a, size_t es);
 // Sequences given with a workspace may leave out what has decayed below kDecayDrop from this length on:
 // at dt near 0.02 the end-state pass of 65536 steps then walks about 1100 of each segment's 4096.
 // Shorter segments hardly reach that decay.
@@ -1807,11 +1808,12 @@ int launch_ps(const ScanArgs& a, const uint16_t* dtlo, const uint16_t* wdt) {
     if (a.ws) {
         nseg = ps_segments(a.Bt, a.Dm, a.L);
         const size_t need = ps_workspace_bytes(a.Bt, a.Dm, a.L);
+        const size_t least = a.ws_may_be_short ? 0 : g_scan_segments > 0 ? need : wave_workspace_bytes(a, sizeof(T));
+        HX_REQUIRE(least == 0 || (a.ws_bytes >= least && aligned(a.ws, 16)), HX_ERR_INVALID_INPUT,
+                   "selective scan: workspace of %zu bytes (16-byte aligned) needed, %zu given "
+                   "(hx_selective_scan_workspace_size)", least, a.ws_bytes);
         if (a.ws_bytes < need || !aligned(a.ws, 16)) {
-            // a workspace too small for a long sequence is refused; elsewhere as many segments as fit
-            HX_REQUIRE(g_scan_segments == 0 && (a.L < 4096 || a.ws_may_be_short), HX_ERR_INVALID_INPUT,
-                       "selective scan: workspace of %zu bytes (16-byte aligned) needed, %zu given "
-                       "(hx_selective_scan_workspace_size)", need, a.ws_bytes);
+            // as many segments as fit
             nseg = aligned(a.ws, 16) ? 1 + (int64_t)(a.ws_bytes / ps_seg_bytes(a.Bt, a.Dm, 2)) : 1;
         }
     }
@@ -2075,17 +2077,23 @@ int run_scan(const ScanArgs& a) {
     return dispatch_fast<T, 8, 16>(a);
 }
 
+// The wave path's workspace for these sizes: a given workspace is refused below it, so that programs
+// that keep one keep their answers whichever kernel runs.
+size_t wave_workspace_bytes(const ScanArgs& a, size_t es) {
+    int64_t seg_len = 0;
+    if (a.Dm % 4 != 0 || (g_scan_variant == 0 && ws_preferred(a, es))) return 0;
+    return scan_seg_bytes(a.Bt, a.Dm, scan_segments(a, &seg_len));
+}
+
 // Workspace bytes the dispatch of run_scan would use for these sizes (pointers assumed aligned;
 // a path that needs none leaves a given workspace unused).
 size_t scan_workspace_bytes(const ScanArgs& a, size_t es) {
     const int v = g_scan_variant;
-    if (a.N == 16 && v == 0 && a.L > 0 && a.Bt > 0 && a.Dm > 0 && ps_ok(a.Bt, a.Dm, a.L, es))
-        return ps_workspace_bytes(a.Bt, a.Dm, a.L);
-    if (a.N != 16 || a.Dm % 4 != 0 || a.L <= 0 || a.Bt <= 0 || a.Dm <= 0) return 0;
+    if (a.N != 16 || a.L <= 0 || a.Bt <= 0 || a.Dm <= 0) return 0;
     if (v != 0 && v != 40 && v != 42) return 0;  // generic, fast and warp-specialised: none
-    if (v == 0 && ws_preferred(a, es)) return 0;
-    int64_t seg_len = 0;
-    return scan_seg_bytes(a.Bt, a.Dm, scan_segments(a, &seg_len));
+    const size_t wave = wave_workspace_bytes(a, es);
+    const size_t ps = v == 0 && ps_ok(a.Bt, a.Dm, a.L, es) ? ps_workspace_bytes(a.Bt, a.Dm, a.L) : 0;
+    return ps > wave ? ps : wave;
 }
 
 int check_common(int64_t Bt, int64_t L, int64_t Dm, int64_t N, int dtype) {
