@@ -717,14 +717,13 @@ __global__ __launch_bounds__(128) void s4d_complex_kernel(
 // The state is kept rescaled, g = h / Bbar, so the update needs no per-state input product:
 //   g_t = Abar*g_{t-1} + u_t,  Re(C*h_t) = Re((C*Bbar)*g_t).
 // Long sequences are cut into time segments (one block each): END_ONLY blocks run a segment from
-// zero and publish its end state; a carry kernel chains entry states (the system is
-// time-invariant, so a segment's transfer is Abar^seg_len); full blocks rerun each segment from
-// its entry state and write y.
+// zero and publish its end state; full blocks chain the segments before their own (the system is
+// time-invariant, so a segment's transfer is Abar^seg_len), rerun it from that entry state and write y.
 struct S4dSeg {
     int64_t seg_len;
     int nseg;
-    const float* seg_init;  // [nseg][Bt][Dm][16][2] entry g (full mode, nseg > 1)
-    float* seg_end;         // [nseg][Bt][Dm][16][2] end g from zero (END_ONLY)
+    bool whole;             // END_ONLY walks whole segments
+    float* seg_end;         // [nseg - 1][Bt][Dm][16][2] end g from zero
 };
 
 __device__ inline void s4d_coef(float dt, float are, float aim, float& ar, float& ai) {
@@ -772,7 +771,6 @@ __global__ __launch_bounds__(256) void s4d_wave_kernel(
 
     float ar[4], ai[4], cr[4], ci[4], gr[4], gi[4];
     const float dt = dtv[dc];
-    const float* g0 = (!END_ONLY && sg.nseg > 1) ? sg.seg_init + (int64_t)seg * Bt * Dm * NS * 2 : nullptr;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const int64_t idx = dc * NS + 4 * r + k;
@@ -780,9 +778,41 @@ __global__ __launch_bounds__(256) void s4d_wave_kernel(
         const float br = dt * B_re[idx], bi = dt * B_im[idx];
         cr[k] = C_re[idx] * br - C_im[idx] * bi;  // C * Bbar
         ci[k] = C_re[idx] * bi + C_im[idx] * br;
-        const int64_t gidx = ((b * Dm + dc) * NS + 4 * r + k) * 2;
-        gr[k] = g0 ? g0[gidx] : 0.0f;
-        gi[k] = g0 ? g0[gidx + 1] : 0.0f;
+        gr[k] = gi[k] = 0.0f;
+    }
+    if constexpr (!END_ONLY) {
+        if (seg > 0) {
+            float pr[4], pi[4];  // Abar^seg_len
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float br = ar[k], bi = ai[k];
+                pr[k] = 1.0f;
+                pi[k] = 0.0f;
+                for (int64_t e = sg.seg_len; e > 0; e >>= 1) {
+                    if (e & 1) {
+                        const float t = pr[k] * br - pi[k] * bi;
+                        pi[k] = pr[k] * bi + pi[k] * br;
+                        pr[k] = t;
+                    }
+                    const float t = br * br - bi * bi;
+                    bi = 2.0f * br * bi;
+                    br = t;
+                }
+            }
+            const float4* ge = reinterpret_cast<const float4*>(sg.seg_end) + ((b * Dm + dc) * NS + 4 * r) / 2;
+            const int64_t per = Bt * Dm * (NS / 2);
+#pragma unroll 8
+            for (int k = 0; k < seg; ++k) {
+                const float4 e0 = ge[k * per], e1 = ge[k * per + 1];
+                const float er[4] = {e0.x, e0.z, e1.x, e1.z}, ei[4] = {e0.y, e0.w, e1.y, e1.w};
+#pragma unroll
+                for (int n = 0; n < 4; ++n) {
+                    const float nr = fmaf(pr[n], gr[n], fmaf(-pi[n], gi[n], er[n]));
+                    gi[n] = fmaf(pr[n], gi[n], fmaf(pi[n], gr[n], ei[n]));
+                    gr[n] = nr;
+                }
+            }
+        }
     }
     const float Dd = Dv ? Dv[dc] : 0.0f;
 
@@ -808,7 +838,7 @@ __global__ __launch_bounds__(256) void s4d_wave_kernel(
         atomicMax(&s_win, dvalid ? wl : 0);
         lds_barrier();
         const int64_t win = s_win;
-        if (win < tend - tbeg) tstart = tend - (win + TCH - 1) / TCH * TCH;
+        if (!sg.whole && win < tend - tbeg) tstart = tend - (win + TCH - 1) / TCH * TCH;
     }
 
     // prefetch ring of PF = 2 chunks in two named registers (an indexed array of float4 was
@@ -903,42 +933,6 @@ __global__ __launch_bounds__(256) void s4d_wave_kernel(
             ge[gidx] = gr[k];
             ge[gidx + 1] = gi[k];
         }
-    }
-}
-
-// Entry g of every segment, per (b, d, n): g_in[0] = 0, g_in[k] = Abar^seg_len * g_in[k-1] +
-// g_end[k-1]. Abar is formed exactly as in s4d_wave_kernel and raised by binary powering.
-__global__ __launch_bounds__(256) void s4d_seg_carry_kernel(
-    int64_t Bt, int64_t Dm, int nseg, int64_t seg_len, const float* __restrict__ dtv,
-    const float* __restrict__ a_re, const float* __restrict__ a_im,
-    const float* __restrict__ gend, float* __restrict__ ginit) {
-    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t per = Bt * Dm * 16;
-    if (gid >= per) return;
-    const int64_t dn = gid % (Dm * 16);
-    const int64_t dd = dn / 16;
-    float br, bi;
-    s4d_coef(dtv[dd], a_re[dn], a_im[dn], br, bi);
-    float pr = 1.0f, pi = 0.0f;  // Abar^seg_len
-    for (int64_t e = seg_len; e > 0; e >>= 1) {
-        if (e & 1) {
-            const float t = pr * br - pi * bi;
-            pi = pr * bi + pi * br;
-            pr = t;
-        }
-        const float t = br * br - bi * bi;
-        bi = 2.0f * br * bi;
-        br = t;
-    }
-    float hr = 0.0f, hi = 0.0f;
-    for (int k = 0; k < nseg; ++k) {
-        const int64_t o = ((int64_t)k * per + gid) * 2;
-        ginit[o] = hr;
-        ginit[o + 1] = hi;
-        const float nr = fmaf(pr, hr, fmaf(-pi, hi, gend[o]));
-        const float ni = fmaf(pr, hi, fmaf(pi, hr, gend[o + 1]));
-        hr = nr;
-        hi = ni;
     }
 }
 
@@ -1333,9 +1327,31 @@ namespace {
 thread_local int g_s4d_path = 0;  // per calling thread (hx_set_s4d_path)
 thread_local int g_s4d_segments = 0;  // per calling thread (hx_set_s4d_segments)
 
-// Time segments of the S4D wave path: about 2048 waves (two per SIMD), segments of at least 512
-// steps, 16-step aligned. Returns the segment count and sets seg_len.
+// Time segments of the S4D wave path, 16-step aligned: two blocks per CU (1 x 65536 x 2048: 474 us with
+// 16, 632 with 8, 476 with 32), at least 64 steps each and at most sqrt(L) / 2 of them, as each one chains
+// those before it (1 x 16384 x 256: 60 us with 64, 78 with 32, 88 with 128). Segments of at least 512
+// steps, the rule before, left short sequences of few channels on a handful of blocks: 1 x 4096 x 64
+// 71 us with 8, 35 with 32; 2 x 2000 x 300 104 with 2, 30 with 25; 3 x 1000 x 2048 76 with 1, 48 with 5. Below
+// 320 steps the second launch costs what the shorter chain saves (1 x 256 x 128: 23 us with 1, 22 with 4).
+// Returns the segment count and sets seg_len.
 int64_t s4d_segments(int64_t Bt, int64_t L, int64_t Dm, int64_t* seg_len_out) {
+    const int64_t pairs = (int64_t)((Dm + 63) / 64) * Bt;
+    int64_t nseg = g_s4d_segments;
+    if (nseg <= 0) {
+        nseg = (512 + pairs - 1) / pairs;
+        const int64_t cap = L >= 320 ? L / 64 : 1;
+        nseg = nseg < cap ? nseg : cap;
+        while (nseg > 1 && 4 * nseg * nseg > L) --nseg;
+    }
+    int64_t seg_len = (L + nseg - 1) / nseg;
+    seg_len = (seg_len + 15) / 16 * 16;
+    *seg_len_out = seg_len;
+    return (L + seg_len - 1) / seg_len;
+}
+// Segments of at least 512 steps, two waves per SIMD: end states that decay inside such a segment start
+// late in it, and their room (end and entry states) is what a given workspace must have. Sequences that
+// these leave whole need no workspace, and their end states leave nothing out.
+int64_t s4d_long_segments(int64_t Bt, int64_t L, int64_t Dm) {
     const int64_t pairs = (int64_t)((Dm + 63) / 64) * Bt;
     int64_t nseg = g_s4d_segments;
     if (nseg <= 0) {
@@ -1343,39 +1359,42 @@ int64_t s4d_segments(int64_t Bt, int64_t L, int64_t Dm, int64_t* seg_len_out) {
         const int64_t cap = L / 512 > 1 ? L / 512 : 1;
         nseg = nseg < cap ? nseg : cap;
     }
-    int64_t seg_len = (L + nseg - 1) / nseg;
-    seg_len = (seg_len + 15) / 16 * 16;
-    *seg_len_out = seg_len;
+    const int64_t seg_len = ((L + nseg - 1) / nseg + 15) / 16 * 16;
     return (L + seg_len - 1) / seg_len;
 }
 bool s4d_wave_ok(int64_t dim, int64_t dstate, const float* x, const float* y) {
     return dstate == 16 && dim % 4 == 0 && aligned(x, 16) && aligned(y, 16) && g_s4d_path != 1;
 }
-// Segment end and entry states, [nseg][B][D][16] complex each.
-size_t s4d_ws_bytes(int64_t Bt, int64_t Dm, int64_t nseg) {
-    return nseg > 1 ? 2 * (size_t)nseg * Bt * Dm * 16 * 2 * sizeof(float) : 0;
+// Bytes of one segment's end states, [B][D][16] complex.
+size_t s4d_seg_bytes(int64_t Bt, int64_t Dm) { return (size_t)Bt * Dm * 16 * 2 * sizeof(float); }
+size_t s4d_least_bytes(int64_t Bt, int64_t L, int64_t Dm) {
+    const int64_t nseg = s4d_long_segments(Bt, L, Dm);
+    return nseg > 1 ? 2 * nseg * s4d_seg_bytes(Bt, Dm) : 0;
+}
+size_t s4d_ws_bytes(int64_t Bt, int64_t L, int64_t Dm) {
+    int64_t seg_len = 0;
+    const size_t need = (s4d_segments(Bt, L, Dm, &seg_len) - 1) * s4d_seg_bytes(Bt, Dm), least = s4d_least_bytes(Bt, L, Dm);
+    return need > least ? need : least;
 }
 
 int launch_s4d_wave(int64_t Bt, int64_t L, int64_t Dm, const float* x, const float* dt,
                     const float* a_re, const float* a_im, const float* B_re, const float* B_im,
                     const float* C_re, const float* C_im, const float* D, float* y,
-                    float* scratch, hipStream_t s) {
+                    float* scratch, size_t scratch_bytes, hipStream_t s) {
     const int ntiles = (int)((Dm + 63) / 64);
     const int64_t pairs = (int64_t)ntiles * Bt;
-    int64_t seg_len = 0;
-    const int64_t nseg = s4d_segments(Bt, L, Dm, &seg_len);
-    HX_REQUIRE(pairs * nseg <= 0x7fffffff, HX_ERR_UNSUPPORTED, "s4d_complex: grid too large");
-    S4dSeg sg{seg_len, (int)nseg, nullptr, nullptr};
-    if (nseg > 1) {
-        const size_t per = (size_t)nseg * Bt * Dm * 16 * 2;
-        sg.seg_end = scratch;
-        sg.seg_init = scratch + per;
-        hipLaunchKernelGGL(s4d_wave_kernel<true>, dim3((unsigned)(pairs * nseg)), dim3(256), 0, s, L,
-                           Dm, ntiles, Bt, x, dt, a_re, a_im, B_re, B_im, C_re, C_im, D, y, sg);
-        const int64_t n = Bt * Dm * 16;
-        hipLaunchKernelGGL(s4d_seg_carry_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                           Bt, Dm, (int)nseg, seg_len, dt, a_re, a_im, sg.seg_end, scratch + per);
+    int64_t seg_len = L;
+    int64_t nseg = s4d_segments(Bt, L, Dm, &seg_len);
+    const int64_t room = scratch && aligned(scratch, 16) ? 1 + (int64_t)(scratch_bytes / s4d_seg_bytes(Bt, Dm)) : 1;
+    if (nseg > room) {  // as many as fit
+        seg_len = ((L + room - 1) / room + 15) / 16 * 16;
+        nseg = (L + seg_len - 1) / seg_len;
     }
+    HX_REQUIRE(pairs * nseg <= 0x7fffffff, HX_ERR_UNSUPPORTED, "s4d_complex: grid too large");
+    const S4dSeg sg{seg_len, (int)nseg, s4d_long_segments(Bt, L, Dm) == 1, scratch};
+    if (nseg > 1)
+        hipLaunchKernelGGL(s4d_wave_kernel<true>, dim3((unsigned)(pairs * (nseg - 1))), dim3(256), 0, s, L,
+                           Dm, ntiles, Bt, x, dt, a_re, a_im, B_re, B_im, C_re, C_im, D, y, sg);
     hipLaunchKernelGGL(s4d_wave_kernel<false>, dim3((unsigned)(pairs * nseg)), dim3(256), 0, s, L,
                        Dm, ntiles, Bt, x, dt, a_re, a_im, B_re, B_im, C_re, C_im, D, y, sg);
     HX_LAUNCH_CHECK();
@@ -1401,8 +1420,7 @@ extern "C" size_t hx_s4d_workspace_size(int64_t batch, int64_t seqlen, int64_t d
     using namespace hx;
     if (batch <= 0 || seqlen <= 0 || dim <= 0 || dstate != 16 || dim % 4 != 0 || g_s4d_path == 1)
         return 0;
-    int64_t seg_len = 0;
-    return s4d_ws_bytes(batch, dim, s4d_segments(batch, seqlen, dim, &seg_len));
+    return s4d_ws_bytes(batch, seqlen, dim);
 }
 
 extern "C" int hx_s4d_complex_fwd(int64_t batch, int64_t seqlen, int64_t dim, int64_t dstate,
@@ -1420,14 +1438,13 @@ extern "C" int hx_s4d_complex_fwd(int64_t batch, int64_t seqlen, int64_t dim, in
                "s4d_complex: a required pointer is NULL");
     hipStream_t s = as_stream(stream);
     if (s4d_wave_ok(dim, dstate, x, y)) {
-        int64_t seg_len = 0;
-        const size_t need = s4d_ws_bytes(batch, dim, s4d_segments(batch, seqlen, dim, &seg_len));
+        const size_t need = s4d_least_bytes(batch, seqlen, dim);
         HX_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned(workspace, 16)),
                    HX_ERR_INVALID_INPUT,
                    "s4d_complex: workspace of %zu bytes (16-byte aligned) needed, %zu given "
                    "(hx_s4d_workspace_size)", need, workspace ? workspace_bytes : (size_t)0);
         return launch_s4d_wave(batch, seqlen, dim, x, dt, a_re, a_im, B_re, B_im, C_re, C_im, D, y,
-                               (float*)workspace, s);
+                               (float*)workspace, workspace_bytes, s);
     }
     const int64_t total = batch * dim;
     dim3 grid((unsigned)((total + 127) / 128));

@@ -223,6 +223,33 @@ def test_s4d_wave_path(dev, bt, L, dim, nseg):
     assert err <= TOL_F32, err
 
 
+@pytest.mark.parametrize("bt,L,dim", [(1, 319, 64), (1, 320, 4), (2, 700, 36), (1, 512, 512), (1, 1023, 68),
+                                      (1, 4099, 64), (5, 2000, 300)])
+def test_s4d_automatic_segments(dev, bt, L, dim):
+    """Sequences of few channels are cut by themselves, on both sides of the shortest that is (320 steps), with
+    ragged last segments and channel tiles; without a workspace they stay whole where none was ever
+    needed (below 1024 steps). A NaN reaches every later output of its channel and no other's."""
+    x, p = s4d_inputs(bt, L, dim, 16, seed=L + dim)
+    kw = {k: dv(v, dev) for k, v in p.items()}
+    r = oracle.s4d_complex(x, **p)
+    from helixml_amd import _ffi
+    assert (_ffi.lib().hx_s4d_workspace_size(bt, L, dim, 16) > 0) == (L >= 320)
+    assert rel_err(ssm.s4d_complex_fwd(dv(x, dev), **kw).cpu().numpy(), r) <= TOL_F32
+    if L >= 1024:
+        return
+    xd = dv(x, dev)
+    y = torch.full_like(xd, float("nan"))
+    _ffi.call("hx_s4d_complex_fwd", bt, L, dim, 16, xd.data_ptr(),
+              *[kw[k].data_ptr() for k in ("dt", "a_re", "a_im", "B_re", "B_im", "C_re", "C_im", "D")],
+              y.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rel_err(y.cpu().numpy(), r) <= TOL_F32
+    kw["a_re"] = kw["a_re"] * 20  # |Abar| = exp(-1): 2^-32 within 23 steps
+    xd[0, 2, 1] = float("nan")
+    bad = torch.isnan(ssm.s4d_complex_fwd(xd, **kw)).cpu().numpy()
+    assert bad[0, 2:, 1].all() and bad.sum() == L - 2
+
+
 @pytest.mark.parametrize("slow_channel", [False, True])
 def test_s4d_segment_decay_window(dev, slow_channel):
     """2048-step segments with |Abar| = exp(-0.05): the end-state pass starts ~450 steps before a
