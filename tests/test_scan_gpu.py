@@ -483,3 +483,21 @@ def test_scan_automatic_segments_keep_non_finite_values(dev, value):
     assert not np.isfinite(out[0, 2:, 7]).any() and not np.isfinite(last[0, 7]).any()
     other = np.arange(64) != 7
     assert np.isfinite(out[0][:, other]).all() and np.isfinite(out[0, :2, 7]).all()
+
+
+def test_scan_kept_workspace_of_the_wave_path(dev):
+    """From 4096 steps a workspace of the wave path's size (here 4 segments' end states, entry states and
+    decays) is enough also where the automatic kernel would use more: fewer segments, the same answer."""
+    bt, L, dim = 1, 4096, 1536
+    x = scan_inputs(bt, L, dim, 16, seed=9)
+    nbytes = 4 * 3 * dim * 16 * 4
+    assert nbytes < ssm.selective_scan_workspace_size(bt, L, dim, 16)
+    from helixml_amd import _ffi
+    d = {k: to_dev(v, dev) for k, v in x.items()}
+    out = torch.full_like(d["u"], float("nan"))
+    ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    _ffi.call("hx_selective_scan_fwd_ws", bt, L, dim, 16, _ffi.HX_F32, 1,
+              *[d[k].data_ptr() if d[k] is not None else None for k in ("u", "delta", "A", "B", "C", "D", "z", "dt_bias")],
+              out.data_ptr(), None, None, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rel_err(out.cpu().numpy(), run_gpu(x, dev)) <= TOL_F32
