@@ -734,7 +734,8 @@ __device__ inline void s4d_coef(float dt, float are, float aim, float& ar, float
     ai = mag * sn;
 }
 
-template <bool END_ONLY>
+// VEC: 16-byte loads and stores (dim % 4 == 0, x and y 16-byte aligned); otherwise 4-byte ones.
+template <bool END_ONLY, bool VEC>
 __global__ __launch_bounds__(256) void s4d_wave_kernel(
     int64_t L, int64_t Dm, int ntiles, int64_t Bt, const float* __restrict__ x,
     const float* __restrict__ dtv, const float* __restrict__ a_re, const float* __restrict__ a_im,
@@ -848,7 +849,14 @@ __global__ __launch_bounds__(256) void s4d_wave_kernel(
     auto fetch = [&](float4& dst, int64_t t0) __attribute__((always_inline)) {
         int64_t t = t0 + mrow;
         t = t < Lm1 ? t : Lm1;
-        dst = *reinterpret_cast<const float4*>(x + rowbase + t * Dm + (mvalid ? mch : 0));
+        const float* row = x + rowbase + t * Dm;
+        if constexpr (VEC) {
+            dst = *reinterpret_cast<const float4*>(row + (mvalid ? mch : 0));
+        } else {
+            const int64_t last = Dm - 1;
+            dst = make_float4(row[mch < last ? mch : last], row[mch + 1 < last ? mch + 1 : last],
+                              row[mch + 2 < last ? mch + 2 : last], row[mch + 3 < last ? mch + 3 : last]);
+        }
     };
     auto stage_in = [&](const float4& src, int buf) __attribute__((always_inline)) {
         *reinterpret_cast<float4*>(&s_x[buf][mrow][mcl]) = src;
@@ -858,8 +866,15 @@ __global__ __launch_bounds__(256) void s4d_wave_kernel(
             const int64_t t = t0 + mrow;
             if (mvalid && t < tend) {
                 const float4 v = *reinterpret_cast<const float4*>(&s_out[buf][mrow][mcl]);
-                __builtin_nontemporal_store(hx_f32x4s{v.x, v.y, v.z, v.w},
-                                            reinterpret_cast<hx_f32x4s*>(y + rowbase + t * Dm + mch));
+                float* dst = y + rowbase + t * Dm + mch;
+                if constexpr (VEC) {
+                    __builtin_nontemporal_store(hx_f32x4s{v.x, v.y, v.z, v.w}, reinterpret_cast<hx_f32x4s*>(dst));
+                } else {
+                    dst[0] = v.x;
+                    if (mch + 1 < Dm) dst[1] = v.y;
+                    if (mch + 2 < Dm) dst[2] = v.z;
+                    if (mch + 3 < Dm) dst[3] = v.w;
+                }
             }
         }
     };
@@ -1362,9 +1377,11 @@ int64_t s4d_long_segments(int64_t Bt, int64_t L, int64_t Dm) {
     const int64_t seg_len = ((L + nseg - 1) / nseg + 15) / 16 * 16;
     return (L + seg_len - 1) / seg_len;
 }
-bool s4d_wave_ok(int64_t dim, int64_t dstate, const float* x, const float* y) {
-    return dstate == 16 && dim % 4 == 0 && aligned(x, 16) && aligned(y, 16) && g_s4d_path != 1;
-}
+bool s4d_wave_ok(int64_t dstate) { return dstate == 16 && g_s4d_path != 1; }
+// Whether rows take 16-byte accesses. The others, with 4-byte ones, against one thread a channel over the
+// whole sequence, which took them before: 1 x 100 x 65 23 us against 49, 2 x 2000 x 301 34 against 819,
+// 1 x 65536 x 2047 0.91 ms against 44.6. They need no workspace and leave nothing out.
+bool s4d_vec_ok(int64_t dim, const float* x, const float* y) { return dim % 4 == 0 && aligned(x, 16) && aligned(y, 16); }
 // Bytes of one segment's end states, [B][D][16] complex.
 size_t s4d_seg_bytes(int64_t Bt, int64_t Dm) { return (size_t)Bt * Dm * 16 * 2 * sizeof(float); }
 size_t s4d_least_bytes(int64_t Bt, int64_t L, int64_t Dm) {
@@ -1373,7 +1390,8 @@ size_t s4d_least_bytes(int64_t Bt, int64_t L, int64_t Dm) {
 }
 size_t s4d_ws_bytes(int64_t Bt, int64_t L, int64_t Dm) {
     int64_t seg_len = 0;
-    const size_t need = (s4d_segments(Bt, L, Dm, &seg_len) - 1) * s4d_seg_bytes(Bt, Dm), least = s4d_least_bytes(Bt, L, Dm);
+    const size_t need = (s4d_segments(Bt, L, Dm, &seg_len) - 1) * s4d_seg_bytes(Bt, Dm);
+    const size_t least = Dm % 4 == 0 ? s4d_least_bytes(Bt, L, Dm) : 0;
     return need > least ? need : least;
 }
 
@@ -1391,12 +1409,14 @@ int launch_s4d_wave(int64_t Bt, int64_t L, int64_t Dm, const float* x, const flo
         nseg = (L + seg_len - 1) / seg_len;
     }
     HX_REQUIRE(pairs * nseg <= 0x7fffffff, HX_ERR_UNSUPPORTED, "s4d_complex: grid too large");
-    const S4dSeg sg{seg_len, (int)nseg, s4d_long_segments(Bt, L, Dm) == 1, scratch};
-    if (nseg > 1)
-        hipLaunchKernelGGL(s4d_wave_kernel<true>, dim3((unsigned)(pairs * (nseg - 1))), dim3(256), 0, s, L,
-                           Dm, ntiles, Bt, x, dt, a_re, a_im, B_re, B_im, C_re, C_im, D, y, sg);
-    hipLaunchKernelGGL(s4d_wave_kernel<false>, dim3((unsigned)(pairs * nseg)), dim3(256), 0, s, L,
-                       Dm, ntiles, Bt, x, dt, a_re, a_im, B_re, B_im, C_re, C_im, D, y, sg);
+    const bool vec = s4d_vec_ok(Dm, x, y);
+    const S4dSeg sg{seg_len, (int)nseg, !vec || s4d_long_segments(Bt, L, Dm) == 1, scratch};
+    auto run = [&](auto kernel, int64_t segs) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(pairs * segs)), dim3(256), 0, s, L, Dm, ntiles, Bt, x, dt,
+                           a_re, a_im, B_re, B_im, C_re, C_im, D, y, sg);
+    };
+    if (nseg > 1) vec ? run(s4d_wave_kernel<true, true>, nseg - 1) : run(s4d_wave_kernel<true, false>, nseg - 1);
+    vec ? run(s4d_wave_kernel<false, true>, nseg) : run(s4d_wave_kernel<false, false>, nseg);
     HX_LAUNCH_CHECK();
     return HX_OK;
 }
@@ -1418,7 +1438,7 @@ extern "C" int hx_set_s4d_segments(int nseg) {
 
 extern "C" size_t hx_s4d_workspace_size(int64_t batch, int64_t seqlen, int64_t dim, int64_t dstate) {
     using namespace hx;
-    if (batch <= 0 || seqlen <= 0 || dim <= 0 || dstate != 16 || dim % 4 != 0 || g_s4d_path == 1)
+    if (batch <= 0 || seqlen <= 0 || dim <= 0 || dstate != 16 || g_s4d_path == 1)
         return 0;
     return s4d_ws_bytes(batch, seqlen, dim);
 }
@@ -1437,8 +1457,8 @@ extern "C" int hx_s4d_complex_fwd(int64_t batch, int64_t seqlen, int64_t dim, in
     HX_REQUIRE(x && dt && a_re && a_im && B_re && B_im && C_re && C_im && y, HX_ERR_INVALID_INPUT,
                "s4d_complex: a required pointer is NULL");
     hipStream_t s = as_stream(stream);
-    if (s4d_wave_ok(dim, dstate, x, y)) {
-        const size_t need = s4d_least_bytes(batch, seqlen, dim);
+    if (s4d_wave_ok(dstate)) {
+        const size_t need = s4d_vec_ok(dim, x, y) ? s4d_least_bytes(batch, seqlen, dim) : 0;
         HX_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned(workspace, 16)),
                    HX_ERR_INVALID_INPUT,
                    "s4d_complex: workspace of %zu bytes (16-byte aligned) needed, %zu given "

@@ -192,8 +192,8 @@ int hx_s4_ref_fwd_parallel(int64_t d_model, int64_t dstate, int64_t seqlen, floa
  *   Abar[d,n] = exp(dt[d]*(a_re[d,n] + i*a_im[d,n])), Bbar = dt[d]*B[d,n] (complex)
  *   h[d,n] = Abar*h + Bbar*x[b,t,d];  y[b,t,d] = 2*Re(sum_n C[d,n]*h[d,n]) + D[d]*x[b,t,d]
  * x, y: [batch, seqlen, dim] fp32. a_re, a_im, B_re, B_im, C_re, C_im: [dim, dstate]; dt, D: [dim].
- * workspace: at least hx_s4d_workspace_size(...) bytes (segment states of the long-sequence
- * path; 0 when the sequence is not segmented), 16-byte aligned. */
+ * workspace: at least hx_s4d_workspace_size(...) bytes (segment states; 0 when the sequence is not
+ * segmented), 16-byte aligned. */
 size_t hx_s4d_workspace_size(int64_t batch, int64_t seqlen, int64_t dim, int64_t dstate);
 int hx_s4d_complex_fwd(int64_t batch, int64_t seqlen, int64_t dim, int64_t dstate,
                        const float* x, const float* dt,
@@ -404,9 +404,9 @@ int hx_set_gemm_kernel(int k);
 int hx_set_s4d_path(int path);
 int hx_set_s4d_segments(int nseg);
 /* Number of time segments the long-sequence path splits a scan into, for later calls on the
- * calling thread (0 = automatic: only when the (batch, 64-channel) tiles cannot fill the GPU and
- * seqlen >= 4096). Segments are scanned in parallel from a zero state, their entry states chained
- * by a carry kernel, then rescanned with outputs. A measurement knob; results agree within fp32
+ * calling thread (0 = automatic: only when the (batch, 64-channel) tiles cannot fill the GPU,
+ * from 512 steps on). Segments are scanned in parallel from a zero state, their entry states
+ * chained, then rescanned with outputs. A measurement knob; results agree within fp32
  * rounding for every setting. */
 int hx_set_scan_segments(int nseg);
 

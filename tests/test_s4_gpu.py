@@ -224,7 +224,8 @@ def test_s4d_wave_path(dev, bt, L, dim, nseg):
 
 
 @pytest.mark.parametrize("bt,L,dim", [(1, 319, 64), (1, 320, 4), (2, 700, 36), (1, 512, 512), (1, 1023, 68),
-                                      (1, 4099, 64), (5, 2000, 300)])
+                                      (1, 4099, 64), (5, 2000, 300),
+                                      (1, 100, 1), (2, 700, 67), (1, 1000, 129), (3, 2000, 62)])  # 4-byte accesses
 def test_s4d_automatic_segments(dev, bt, L, dim):
     """Sequences of few channels are cut by themselves, on both sides of the shortest that is (320 steps), with
     ragged last segments and channel tiles; without a workspace they stay whole where none was ever
@@ -245,9 +246,9 @@ def test_s4d_automatic_segments(dev, bt, L, dim):
     torch.cuda.synchronize()
     assert rel_err(y.cpu().numpy(), r) <= TOL_F32
     kw["a_re"] = kw["a_re"] * 20  # |Abar| = exp(-1): 2^-32 within 23 steps
-    xd[0, 2, 1] = float("nan")
+    xd[0, 2, 0] = float("nan")
     bad = torch.isnan(ssm.s4d_complex_fwd(xd, **kw)).cpu().numpy()
-    assert bad[0, 2:, 1].all() and bad.sum() == L - 2
+    assert bad[0, 2:, 0].all() and bad.sum() == L - 2
 
 
 @pytest.mark.parametrize("slow_channel", [False, True])
