@@ -1796,9 +1796,11 @@ size_t wave_workspace_bytes(const ScanArgs& a, size_t es);
 // at dt near 0.02 the end-state pass of 65536 steps then walks about 1100 of each segment's 4096.
 // Shorter segments hardly reach that decay.
 constexpr int64_t kDropSteps = 4096;
-// scan_ps_kernel's sizes: a segment's byte offsets, a few chunks of read-ahead included, below 2^31.
+// scan_ps_kernel's sizes: a segment's byte offsets, a few chunks of read-ahead included, below 2^31, in the
+// rows of u, delta, z and out (Dm wide) and in those of B and C (16 wide).
 bool ps_ok(int64_t Bt, int64_t Dm, int64_t L, size_t es) {
-    return L < (1LL << 30) && (L + 96) * Dm * (int64_t)es < (1LL << 31) && Bt * ((Dm + 63) / 64) <= 0x7fffffff;
+    const int64_t row = (Dm > 16 ? Dm : 16) * (int64_t)es;
+    return L < (1LL << 30) && (L + 96) * row < (1LL << 31) && Bt * ((Dm + 63) / 64) <= 0x7fffffff;
 }
 
 template <typename T, bool HAS_Z, bool SP, int DTPK>

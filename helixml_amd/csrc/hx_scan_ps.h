@@ -76,7 +76,7 @@ __device__ inline float to_f32(uint16_t v) { return bf16_bits_to_f32(v); }
 // segment instead: a NaN, an infinity or an outlier reaches everything after it, as in the uncut scan,
 // and segments of a few hundred steps hardly ever decay that far. The output pass chains the segments
 // before its own itself.
-// Sizes: byte offsets inside a segment below 2^31.
+// Sizes: byte offsets inside a segment below 2^31, in B and C (16 wide) too.
 template <typename T, bool HAS_Z, bool SOFTPLUS, bool END_ONLY, int DTPK>
 __global__ __launch_bounds__(512, 4) void scan_ps_kernel(
     const PsArgs a, const T* __restrict__ u, const T* __restrict__ delta, const T* __restrict__ Bm,

@@ -65,6 +65,17 @@ def test_scan_null_pointers_rejected():
     assert rc == _ffi.InvalidInput.status
 
 
+@pytest.mark.parametrize("dtype,size", [(_ffi.HX_F32, 4), (_ffi.HX_BF16, 2)])
+@pytest.mark.parametrize("dim", [1, 3, 7, 15, 17, 33])
+def test_scan_paired_kernel_bounds_every_operand(dtype, size, dim):
+    """The automatic scan kernel addresses the rows of u (dim wide) and of B and C (16 wide) with 32-bit byte
+    offsets: it takes a size (and asks for a workspace, which no other kernel does for these dims) only while the
+    wider of the two, 96 steps of read-ahead included, stays below 2^31 bytes."""
+    first = -(-2 ** 31 // (max(dim, 16) * size)) - 96  # the first length past the bound
+    size_of = lambda L: _ffi.lib().hx_selective_scan_workspace_size(1, L, dim, 16, dtype)  # noqa: E731
+    assert size_of(first - 1) > 0 and size_of(first) == 0 and size_of(2 ** 28 + 1) == 0
+
+
 def test_s4_ref_rejects():
     L = _ffi.lib()
     assert L.hx_s4_ref_fwd(4, 0, 4, 0.1, *([None] * 7), None, 0, None) == _ffi.UnsupportedOperation.status
