@@ -1791,11 +1791,22 @@ size_t ps_seg_bytes(int64_t Bt, int64_t Dm, int64_t nseg) {
 size_t ps_workspace_bytes(int64_t Bt, int64_t Dm, int64_t L) {
     return ps_seg_bytes(Bt, Dm, ps_seg_count(L, ps_seg_len(L, ps_segments(Bt, Dm, L))));
 }
+// Whether rows take the wave kernels' 16-byte accesses.
+bool tile_ok(const ScanArgs& a) {
+    return a.Dm % 4 == 0 && aligned(a.u, 16) && aligned(a.delta, 16) && aligned(a.out, 16) &&
+           (!a.z || aligned(a.z, 16)) && (!a.D || aligned(a.D, 16)) && (!a.dt_bias || aligned(a.dt_bias, 16)) &&
+           a.Bt * ((a.Dm + 63) / 64) <= 0x7fffffff;
+}
 size_t wave_workspace_bytes(const ScanArgs& a, size_t es);
-// Sequences given with a workspace may leave out what has decayed below kDecayDrop from this length on:
-// at dt near 0.02 the end-state pass of 65536 steps then walks about 1100 of each segment's 4096.
-// Shorter segments hardly reach that decay.
+// Sequences given with a workspace may leave out what has decayed below kDecayDrop from this length on,
+// where the wave path cuts them too: at dt near 0.02 the end-state pass of 65536 steps then walks about 1100
+// of each segment's 4096. Shorter segments hardly reach that decay. All others walk whole segments, so that
+// a NaN, an infinity or an outlier reaches everything after it.
 constexpr int64_t kDropSteps = 4096;
+template <typename T>
+bool ps_drop(const ScanArgs& a) {
+    return a.L >= kDropSteps && !a.ws_may_be_short && tile_ok(a) && wave_workspace_bytes(a, sizeof(T)) > 0;
+}
 // scan_ps_kernel's sizes: a segment's byte offsets, a few chunks of read-ahead included, below 2^31, in the
 // rows of u, delta, z and out (Dm wide) and in those of B and C (16 wide).
 bool ps_ok(int64_t Bt, int64_t Dm, int64_t L, size_t es) {
@@ -1826,7 +1837,7 @@ int launch_ps(const ScanArgs& a, const uint16_t* dtlo, const uint16_t* wdt) {
     float4* hend = (float4*)a.ws;
     float4* decay = hend + (nseg - 1) * a.Bt * ntiles * 256;
     const PsArgs pa{a.L, a.Dm, (int)ntiles, (int)a.Bt, (int)nseg, (int)seg_len,
-                    a.L >= kDropSteps && !a.ws_may_be_short, a.A, a.D, a.dt_bias,
+                    ps_drop<T>(a), a.A, a.D, a.dt_bias,
                     a.init_state, a.last_state, hend, decay, dtlo, wdt};
     if (nseg > 1) {
         hipLaunchKernelGGL((scan_ps_kernel<T, false, SP, true, DTPK>), dim3((unsigned)(ntiles * a.Bt * (nseg - 1))),
@@ -2037,10 +2048,7 @@ int run_scan(const ScanArgs& a) {
     const bool fast_ok = a.N == 16 && aligned(a.B, 16 * es) && aligned(a.C, 16 * es);
     const int v = g_scan_variant;
     if (!fast_ok || v < 0) return dispatch_generic<T>(a);
-    const bool tile_ok = a.Dm % 4 == 0 && aligned(a.u, 16) && aligned(a.delta, 16) &&
-                         aligned(a.out, 16) && (!a.z || aligned(a.z, 16)) &&
-                         (!a.D || aligned(a.D, 16)) && (!a.dt_bias || aligned(a.dt_bias, 16)) &&
-                         a.Bt * ((a.Dm + 63) / 64) <= 0x7fffffff;
+    const bool tiles = tile_ok(a);
     if (v == 0) {
         // auto: scan_ps_kernel; fp32 that fits one block per CU of the split-state warp-specialised
         // kernel, whose 48-channel blocks spread such a size over a third more CUs than 64-channel
@@ -2049,11 +2057,11 @@ int run_scan(const ScanArgs& a) {
         if (ps_ok(a.Bt, a.Dm, a.L, es)) {
             const bool cut = a.ws && ps_segments(a.Bt, a.Dm, a.L) > 1;
             if constexpr (std::is_same<T, float>::value)
-                if (!cut && tile_ok && ws2_ok<T>(a) && a.Bt * ((a.Dm + 47) / 48) <= device_cus())
+                if (!cut && tiles && ws2_ok<T>(a) && a.Bt * ((a.Dm + 47) / 48) <= device_cus())
                     return dispatch_ws<T, 3, true>(a);
             return dispatch_ps<T>(a);
         }
-        if (tile_ok) {
+        if (tiles) {
             if (ws_preferred(a, sizeof(T))) {
                 // fp32: the split-state form (two waves per SIMD; config 2 132.5 vs 145.4 us).
                 // bf16 keeps the 4-wave form, which measured faster there (154.9 vs 162.1 us).
@@ -2066,13 +2074,13 @@ int run_scan(const ScanArgs& a) {
         return dispatch_fast<T, 8, 16>(a);
     }
     switch (v) {
-        case 40: if (tile_ok) return dispatch_wave<T, 2>(a); break;
-        case 42: if (tile_ok && a.L * a.Dm < (1LL << 31)) return dispatch_wave<T, 2, 3>(a); break;
+        case 40: if (tiles) return dispatch_wave<T, 2>(a); break;
+        case 42: if (tiles && a.L * a.Dm < (1LL << 31)) return dispatch_wave<T, 2, 3>(a); break;
         case 44:
-            if (tile_ok && (a.L + 16) * a.Dm * (int64_t)sizeof(T) < (1LL << 32)) return dispatch_ws<T, 2>(a);
+            if (tiles && (a.L + 16) * a.Dm * (int64_t)sizeof(T) < (1LL << 32)) return dispatch_ws<T, 2>(a);
             break;
         case 46:
-            if (tile_ok && ws2_ok<T>(a)) return dispatch_ws<T, 3, true>(a);
+            if (tiles && ws2_ok<T>(a)) return dispatch_ws<T, 3, true>(a);
             break;
         default: break;
     }

@@ -72,10 +72,10 @@ __device__ inline float to_f32(uint16_t v) { return bf16_bits_to_f32(v); }
 // it walks backwards from the end, adding exp2(A * S) * B*dt*u with S the sum of dt from there to the
 // end, and stops at the first 48-step round at which every state of the block's channels has decayed
 // below 2^-32 (kDecayDrop): what is left out is 2^-8 of the fp32 rounding of the state there. Such a
-// segment publishes decay 0. Below 4096 steps and in the Mamba block (drop = 0) it walks its whole
-// segment instead: a NaN, an infinity or an outlier reaches everything after it, as in the uncut scan,
-// and segments of a few hundred steps hardly ever decay that far. The output pass chains the segments
-// before its own itself.
+// segment publishes decay 0. Below 4096 steps, in the Mamba block, and for dims that are no multiple of 4
+// or rows that are not 16-byte aligned (drop = 0) it walks its whole segment instead: a NaN, an infinity or
+// an outlier reaches everything after it, as in the uncut scan, and segments of a few hundred steps hardly
+// ever decay that far. The output pass chains the segments before its own itself.
 // Sizes: byte offsets inside a segment below 2^31, in B and C (16 wide) too.
 template <typename T, bool HAS_Z, bool SOFTPLUS, bool END_ONLY, int DTPK>
 __global__ __launch_bounds__(512, 4) void scan_ps_kernel(

@@ -470,18 +470,33 @@ def test_scan_workspace_below_the_size_asked_for(dev):
                   ws.data_ptr(), 16, torch.cuda.current_stream().cuda_stream)
 
 
-@pytest.mark.parametrize("value", [float("nan"), float("inf")])
-def test_scan_automatic_segments_keep_non_finite_values(dev, value):
-    """A sequence below 4096 steps that is cut by itself loses no NaN or infinity: one input early in the
-    first segment, with steps so large that its state decays by 2^-1000 before that segment ends, leaves
-    that channel's later outputs without a finite value, as the recurrence does, and no other channel's."""
-    x = scan_inputs(1, 1000, 64, 16, seed=5)
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), 1e30])
+@pytest.mark.parametrize("L,dim,offset", [(1000, 64, 0), (8192, 62, 0), (8192, 65, 0), (8192, 64, 1)])
+def test_scan_automatic_segments_keep_non_finite_values(dev, value, L, dim, offset):
+    """A sequence below 4096 steps that is cut by itself loses no NaN, infinity or outlier, nor does one of any length
+    whose dim is no multiple of 4 or whose rows are not 16-byte aligned: one input early in the first segment, with
+    steps so large that its state decays below 2^-32 before that segment ends. A NaN or an infinity leaves that
+    channel's later outputs without a finite value, as the recurrence does, and no other channel's; the outlier's
+    state, exp(-0.6 * 94) of it by then, still dominates the next segment (float64: steps 96 to 111). That decay's
+    exponent reaches 66, a sum of up to 110 steps whose partial sums are each rounded by 2^-24 of themselves: at
+    most 66 * 110 / 2 * 2^-24 = 2.2e-4 of the state, twice that allowed."""
+    x = scan_inputs(1, L, dim, 16, seed=5)
     x["u"][0, 2, 7] = value
-    x["delta"][:] = 1.0
-    assert ssm.selective_scan_workspace_size(1, 1000, 64, 16) > 0
-    out, last = run_gpu(x, dev, last=True)
+    x["delta"][:] = 0.6 if value == 1e30 else 1.0
+    assert ssm.selective_scan_workspace_size(1, L, dim, 16) > 0
+    d = {k: to_dev(v, dev) for k, v in x.items()}
+    if offset:
+        u = torch.empty(L * dim + 1, device=dev)[1:].view(1, L, dim)
+        d["u"] = u.copy_(d["u"])
+    out, last = ssm.selective_scan_fwd(**d, delta_softplus=False, return_last_state=True)
+    out, last = out.cpu().numpy(), last.cpu().numpy()
+    if value == 1e30:
+        r, _ = oracle.numpy_selective_scan(**x, delta_softplus=False)
+        assert np.abs(r[0, 96, 7]) > 100
+        assert rel_err(out[0, 96:112, 7], r[0, 96:112, 7]) <= 4.4e-4
+        return
     assert not np.isfinite(out[0, 2:, 7]).any() and not np.isfinite(last[0, 7]).any()
-    other = np.arange(64) != 7
+    other = np.arange(dim) != 7
     assert np.isfinite(out[0][:, other]).all() and np.isfinite(out[0, :2, 7]).all()
 
 
