@@ -69,8 +69,9 @@ __device__ inline float to_f32(uint16_t v) { return bf16_bits_to_f32(v); }
 // priority gives 2-3%.
 //
 // END_ONLY: a segment's end state from a zero entry state and its decay, for the segments that follow;
-// it walks backwards from the end, adding exp2(A * S) * B*dt*u with S the sum of dt from there to the
-// end, and stops at the first 48-step round at which every state of the block's channels has decayed
+// it walks backwards from the end, adding exp2(S) * B*dt*u with S the sum of A*dt from there to the end
+// (a sum per state, one FMA each: A = -inf gives S = -inf, where A times a sum of dt would be NaN at the last
+// step, whose sum is 0), and stops at the first 48-step round at which every state of the block's channels has decayed
 // below 2^-32 (kDecayDrop): what is left out is 2^-8 of the fp32 rounding of the state there. Such a
 // segment publishes decay 0. Below 4096 steps, in the Mamba block, and for dims that are no multiple of 4
 // or rows that are not 16-byte aligned (drop = 0) it walks its whole segment instead: a NaN, an infinity or
@@ -213,7 +214,7 @@ __global__ __launch_bounds__(512, 4) void scan_ps_kernel(
         }
         if constexpr (DTP) lds_barrier();
         lds_barrier();
-        float S = 0.0f;  // END_ONLY: sum of dt from the step reached to the segment's end
+        float ex[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // END_ONLY: log2 of each state's decay from the step reached to the segment's end
         bool dropped = false;
         constexpr int G0 = END_ONLY ? 3 : 0;  // first group of 4 steps walked
         float du[4];
@@ -255,11 +256,13 @@ __global__ __launch_bounds__(512, 4) void scan_ps_kernel(
 #pragma unroll
                     for (int e = 3; e >= 0; --e) {
 #pragma unroll
-                        for (int n = 0; n < 4; ++n) h[n] = fmaf(fast_exp2(A2[n] * S), xc[4 * e + n], h[n]);
-                        S += qd[e];
+                        for (int n = 0; n < 4; ++n) {
+                            h[n] = fmaf(fast_exp2(ex[n]), xc[4 * e + n], h[n]);
+                            ex[n] = fmaf(A2[n], qd[e], ex[n]);
+                        }
                     }
                     // nothing here has a side effect: pins the group's work to its place
-                    asm volatile("" : "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]), "+v"(S));
+                    asm volatile("" : "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]), "+v"(ex[0]), "+v"(ex[1]), "+v"(ex[2]), "+v"(ex[3]));
                 } else {
                     float ab[4][4];
 #pragma unroll
@@ -285,9 +288,9 @@ __global__ __launch_bounds__(512, 4) void scan_ps_kernel(
             if constexpr (END_ONLY && k == NB - 1) {
                 // stop once every state of the block's channels has decayed below 2^-32 on its way
                 // to the segment's end (a NaN or growing decay never stops it)
-                float m = fast_exp2(A2[0] * S);
+                float m = fast_exp2(ex[0]);
 #pragma unroll
-                for (int n = 1; n < 4; ++n) m = fmaxf(m, fast_exp2(A2[n] * S));
+                for (int n = 1; n < 4; ++n) m = fmaxf(m, fast_exp2(ex[n]));
                 const int go = __ballot(dvalid && !(m < kDecayDrop)) != 0;
                 if (lane == 0) s_vote[0][w] = go;
             }
@@ -300,7 +303,7 @@ __global__ __launch_bounds__(512, 4) void scan_ps_kernel(
             a.hend[o] = make_float4(h[0], h[1], h[2], h[3]);
             float q[4];
 #pragma unroll
-            for (int n = 0; n < 4; ++n) q[n] = dropped ? 0.0f : fast_exp2(A2[n] * S);
+            for (int n = 0; n < 4; ++n) q[n] = dropped ? 0.0f : fast_exp2(ex[n]);
             a.decay[o] = make_float4(q[0], q[1], q[2], q[3]);
         } else if (a.last && dvalid && seg == a.nseg - 1) {
 #pragma unroll

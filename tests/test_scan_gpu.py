@@ -500,6 +500,22 @@ def test_scan_automatic_segments_keep_non_finite_values(dev, value, L, dim, offs
     assert np.isfinite(out[0][:, other]).all() and np.isfinite(out[0, :2, 7]).all()
 
 
+def test_scan_automatic_segments_state_that_keeps_nothing(dev):
+    """A = -inf (an A_log above 88.7): that state's decay is 0, so each step's state is its own input. A cut
+    sequence gives what the uncut one does."""
+    x = scan_inputs(1, 1008, 70, 16, seed=6)
+    x["A"][7, 3] = -np.inf
+    assert ssm.selective_scan_workspace_size(1, 1008, 70, 16) > 0
+    cut, last = run_gpu(x, dev, last=True)
+    ssm.set_scan_segments(1)
+    try:
+        whole, wlast = run_gpu(x, dev, last=True)
+    finally:
+        ssm.set_scan_segments(0)
+    assert np.isfinite(whole).all() and np.isfinite(wlast).all()
+    assert rel_err(cut, whole) <= TOL_F32 and rel_err(last, wlast) <= TOL_F32
+
+
 def test_scan_kept_workspace_of_the_wave_path(dev):
     """From 4096 steps a workspace of the wave path's size (here 4 segments' end states, entry states and
     decays) is enough also where the automatic kernel would use more: fewer segments, the same answer."""
