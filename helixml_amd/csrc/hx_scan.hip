@@ -1805,7 +1805,7 @@ size_t wave_workspace_bytes(const ScanArgs& a, size_t es);
 constexpr int64_t kDropSteps = 4096;
 template <typename T>
 bool ps_drop(const ScanArgs& a) {
-    return a.L >= kDropSteps && !a.ws_may_be_short && tile_ok(a) && wave_workspace_bytes(a, sizeof(T)) > 0;
+    return a.L >= kDropSteps && !a.ws_may_be_short && wave_workspace_bytes(a, sizeof(T)) > 0;
 }
 // scan_ps_kernel's sizes: a segment's byte offsets, a few chunks of read-ahead included, below 2^31, in the
 // rows of u, delta, z and out (Dm wide) and in those of B and C (16 wide).
@@ -1821,7 +1821,7 @@ int launch_ps(const ScanArgs& a, const uint16_t* dtlo, const uint16_t* wdt) {
     if (a.ws) {
         nseg = ps_segments(a.Bt, a.Dm, a.L);
         const size_t need = ps_workspace_bytes(a.Bt, a.Dm, a.L);
-        const size_t least = a.ws_may_be_short ? 0 : g_scan_segments > 0 ? need : wave_workspace_bytes(a, sizeof(T));
+        const size_t least = a.ws_may_be_short ? 0 : wave_workspace_bytes(a, sizeof(T));
         HX_REQUIRE(least == 0 || (a.ws_bytes >= least && aligned(a.ws, 16)), HX_ERR_INVALID_INPUT,
                    "selective scan: workspace of %zu bytes (16-byte aligned) needed, %zu given "
                    "(hx_selective_scan_workspace_size)", least, a.ws_bytes);
@@ -2087,11 +2087,11 @@ int run_scan(const ScanArgs& a) {
     return dispatch_fast<T, 8, 16>(a);
 }
 
-// The wave path's workspace for these sizes: a given workspace is refused below it, so that programs
+// The wave path's workspace for these sizes and rows: a given workspace is refused below it, so that programs
 // that keep one keep their answers whichever kernel runs.
 size_t wave_workspace_bytes(const ScanArgs& a, size_t es) {
     int64_t seg_len = 0;
-    if (a.Dm % 4 != 0 || (g_scan_variant == 0 && ws_preferred(a, es))) return 0;
+    if (!tile_ok(a) || (g_scan_variant == 0 && ws_preferred(a, es))) return 0;
     return scan_seg_bytes(a.Bt, a.Dm, scan_segments(a, &seg_len));
 }
 

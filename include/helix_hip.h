@@ -102,12 +102,15 @@ int hx_selective_scan_fwd(int64_t batch, int64_t seqlen, int64_t dim, int64_t ds
 /* hx_selective_scan_fwd with a caller workspace for cutting the sequence: when the (batch, channel)
  * tiles alone cannot fill the GPU (few channels and at least some hundred steps), the sequence is
  * cut into time segments whose end states (from a zero state) are accumulated backwards from
- * each segment's end (from 4096 steps on until every state's decay to the end is below 2^-32, which
- * leaves out what came before), and every segment is then scanned with outputs from the chained
- * entry state (results agree with the unsegmented scan to fp32 rounding). workspace: device memory
- * of at least hx_selective_scan_workspace_size(...) bytes, 16-byte aligned (0 bytes: no segments;
- * fewer: below 4096 steps as many segments as fit, from there the call is refused); it holds no
- * state between calls. Same reference
+ * each segment's end, and every segment is then scanned with outputs from the chained entry state
+ * (results agree with the unsegmented scan to fp32 rounding). From 4096 steps on, with dim % 4 == 0 and
+ * 16-byte aligned rows, fewer than 256 (batch, 64-channel) tiles, the accumulation stops once every
+ * state's decay to the segment's end is below 2^-32, which leaves out what came before (a NaN included);
+ * elsewhere it walks whole segments. workspace: device memory of at least
+ * hx_selective_scan_workspace_size(...) bytes, 16-byte aligned (0 bytes: no segments); it holds no state
+ * between calls. With fewer bytes as many segments as fit are used, except that those sequences of
+ * 4096 steps and more refuse a workspace below min(512 / tiles rounded up, seqlen / 1024) segments of
+ * 3 * batch * dim * 64 bytes each (a count of 1 needs none). Same reference
  * counterpart as hx_selective_scan_fwd (the per-step loop of ssm.rs:166-182). */
 size_t hx_selective_scan_workspace_size(int64_t batch, int64_t seqlen, int64_t dim,
                                         int64_t dstate, int dtype);

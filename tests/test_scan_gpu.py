@@ -532,3 +532,26 @@ def test_scan_kept_workspace_of_the_wave_path(dev):
               out.data_ptr(), None, None, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert rel_err(out.cpu().numpy(), run_gpu(x, dev)) <= TOL_F32
+
+
+@pytest.mark.parametrize("dim,offset,segments", [(64, 1, 0), (62, 0, 0), (62, 0, 8)])
+def test_scan_short_workspace_of_rows_that_no_kernel_needed_it_for(dev, dim, offset, segments):
+    """Rows that are not 16-byte aligned, or dims that are no multiple of 4, never needed a workspace: a short one
+    is taken at any length, and with a forced number of segments too."""
+    L = 4100
+    x = scan_inputs(1, L, dim, 16, seed=4)
+    r64, _ = oracle.numpy_selective_scan(**x)
+    from helixml_amd import _ffi
+    d = {k: to_dev(v, dev) for k, v in x.items()}
+    u = torch.empty(L * dim + offset, device=dev)[offset:].view(1, L, dim).copy_(d["u"])
+    out = torch.full((1, L, dim), float("nan"), device=dev)
+    ws = torch.empty(16, device=dev, dtype=torch.uint8)
+    ssm.set_scan_segments(segments)
+    try:
+        _ffi.call("hx_selective_scan_fwd_ws", 1, L, dim, 16, _ffi.HX_F32, 1, u.data_ptr(),
+                  *[d[k].data_ptr() if d[k] is not None else None for k in ("delta", "A", "B", "C", "D", "z", "dt_bias")],
+                  out.data_ptr(), None, None, ws.data_ptr(), 16, torch.cuda.current_stream().cuda_stream)
+    finally:
+        ssm.set_scan_segments(0)
+    torch.cuda.synchronize()
+    assert rel_err(out.cpu().numpy(), r64) <= TOL_F32
