@@ -1513,11 +1513,17 @@ int launch_d256p(int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, co
 bool dlds_ok(size_t bytes) { return hx::grant_dynamic_lds((const void*)hx::gemm_bf16_nt_dlds_kernel, bytes, 0); }
 
 template <int CB>
+bool narrow_ok() {
+    return hx::grant_dynamic_lds((const void*)hx::gemm_bf16_nt_narrow_kernel<CB>,
+                                 (size_t)hx::narrow_stages<CB>() * hx::narrow_stage_bytes<CB>(), 0);
+}
+
+template <int CB>
 int launch_narrow_cb(int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* W,
                      int64_t ldw, const float* bias, const hx::GemmOut& o, void* stream) {
     using namespace hx;
     const size_t bytes = (size_t)narrow_stages<CB>() * narrow_stage_bytes<CB>();
-    HX_REQUIRE(grant_dynamic_lds((const void*)gemm_bf16_nt_narrow_kernel<CB>, bytes, 0), HX_ERR_UNSUPPORTED,
+    HX_REQUIRE(narrow_ok<CB>(), HX_ERR_UNSUPPORTED,
                "gemm_bf16: the device does not grant %zu bytes of LDS", bytes);
     HX_REQUIRE((M + NBM - 1) / NBM <= 0x7fffffff, HX_ERR_UNSUPPORTED, "gemm_bf16: M=%lld too large",
                (long long)M);
@@ -1677,13 +1683,13 @@ extern "C" int hx_gemm_bf16(int64_t M, int64_t N, int64_t K, const void* X, int6
     if (g_gemm_kernel == 0 && vec && K % 8 == 0 && K >= 64 && !small_out) {
         if (K % 64 == 0 && N >= 256 && M >= 256 && ((M + XBM - 1) / XBM) * ((N + XBN - 1) / XBN) >= 112 && d256_ok<64, 2>())
             return launch_d256<64, 2>(M, N, K, X, ldx, W, ldw, bias, o, stream);
-        if ((N + 63) / 64 <= 65535)
-            return ((M + 63) / 64) * ((N + 127) / 128) < 160 ? launch_narrow_cb<1>(M, N, K, X, ldx, W, ldw, bias, o, stream)
-                                                             : launch_narrow_cb<2>(M, N, K, X, ldx, W, ldw, bias, o, stream);
+        const bool one = ((M + 63) / 64) * ((N + 127) / 128) < 160;
+        if ((N + 63) / 64 <= 65535 && (one ? narrow_ok<1>() : narrow_ok<2>()))
+            return one ? launch_narrow_cb<1>(M, N, K, X, ldx, W, ldw, bias, o, stream)
+                       : launch_narrow_cb<2>(M, N, K, X, ldx, W, ldw, bias, o, stream);
     }
     const size_t dlds = (size_t)DSTAGES * DSTAGE_BYTES;
-    if (vec && K > 0 && K % LBK == 0 && g_gemm_kernel == 4 &&
-        dlds_ok(dlds)) {
+    if (vec && K > 0 && K % LBK == 0 && g_gemm_kernel == 4 && dlds_ok(dlds)) {
         dim3 lg((unsigned)((N + LBN - 1) / LBN), (unsigned)((M + LBM - 1) / LBM));
         hipLaunchKernelGGL(gemm_bf16_nt_dlds_kernel, lg, dim3(256), dlds, as_stream(stream), M, N, K,
                            (const uint16_t*)X, ldx, (const uint16_t*)W, ldw, bias, o);

@@ -6,6 +6,7 @@ from pathlib import Path
 
 import numpy as np
 import pytest
+import torch
 
 from helixml_amd import _ffi
 
@@ -74,6 +75,17 @@ def test_scan_paired_kernel_bounds_every_operand(dtype, size, dim):
     first = -(-2 ** 31 // (max(dim, 16) * size)) - 96  # the first length past the bound
     size_of = lambda L: _ffi.lib().hx_selective_scan_workspace_size(1, L, dim, 16, dtype)  # noqa: E731
     assert size_of(first - 1) > 0 and size_of(first) == 0 and size_of(2 ** 28 + 1) == 0
+
+
+@pytest.mark.skipif(torch.cuda.device_count() > 0, reason="launches nothing only where there is no device")
+@pytest.mark.parametrize("M,N,K", [(1999, 768, 1536), (777, 1024, 2048), (4096, 2048, 512)])
+def test_gemm_without_its_lds_falls_through(M, N, K):
+    """Where a device does not grant a kernel its LDS, the automatic choice goes on to one that needs none; it
+    refuses no size for it. Without a device every grant fails, and so does the launch that is reached at last (the
+    operands are never touched)."""
+    p = 4096
+    rc = _ffi.lib().hx_gemm_bf16(M, N, K, p, K, p, K, None, 0, _ffi.HX_BF16, p, N, N, None, 0, N, None, 0, None)
+    assert rc == _ffi.BackendError.status, _ffi.last_error()
 
 
 def test_s4_ref_rejects():
