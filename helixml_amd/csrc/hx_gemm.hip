@@ -751,8 +751,9 @@ constexpr int narrow_stage_bytes() { return (NBM + 64 * CB) * 128; }
 template <int CB>
 constexpr int narrow_stages() { return CB >= 3 ? 4 : 3; }
 
-// What the lanes of a ragged last K tile read past K.
-__device__ const uint16_t kZeros[8] = {};
+// What the lanes of a ragged last K tile read past K, in one 16-byte load.
+alignas(16) __device__ const uint16_t kZeros[8] = {};
+static_assert(__alignof__(kZeros) >= 16, "read by 16-byte loads");
 
 template <int CB>
 __global__ __launch_bounds__(256) void gemm_bf16_nt_narrow_kernel(int64_t M, int64_t N, int64_t K,
