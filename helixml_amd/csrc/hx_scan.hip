@@ -2158,6 +2158,7 @@ int scan_fwd_scratch(int64_t batch, int64_t seqlen, int64_t dim, const uint16_t*
                      const float* A, const uint16_t* B, const uint16_t* C, const float* D, const uint16_t* z,
                      const float* dt_bias, uint16_t* out, float* last_state, void* ws, size_t ws_bytes,
                      hipStream_t stream) {
+    if (int rc = check_common(batch, seqlen, dim, 16, HX_BF16)) return rc;
     ScanArgs a{batch, seqlen, dim, 16, 1, u, delta, A, B, C, D, z, dt_bias, out, nullptr, last_state, stream};
     if (g_scan_variant == 0 && g_scan_segments == 0 && ps_ok(batch, dim, seqlen, 2)) {
         a.ws = ws;

@@ -148,6 +148,11 @@ def test_mamba_block_errors(dev):
     p8 = to_dev(block_inputs(1, 8, 16, 32, 8, 8, 4, seed=1), dev)
     with pytest.raises(UnsupportedOperation):
         ssm.mamba_block_fwd(**p8)
+    # more sequences than the scan takes, with and without dt_proj inside it
+    for r in (8, 32):
+        many = dict(to_dev(block_inputs(1, 8, 16, 32, 16, r, 4, seed=1), dev), x=torch.zeros((65536, 1, 16), device=dev, dtype=BF))
+        with pytest.raises(UnsupportedOperation):
+            ssm.mamba_block_fwd(**many)
 
 
 def test_mamba_block_config3_full_size(dev):
