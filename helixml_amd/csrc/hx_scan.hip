@@ -1762,20 +1762,26 @@ size_t scan_seg_bytes(int64_t Bt, int64_t Dm, int64_t nseg) {
     return (size_t)nseg * 3 * per * sizeof(float);
 }
 
-// Time segments of scan_ps_kernel for Bt x Dm channels. At most 128 (batch, 64-channel) tiles leave
-// half of the 256 CUs idle, and cutting the sequence costs a second, cheaper pass over it (1.75 times
-// the work at most): worth it from there. One block per CU measured best (24 tiles x 2048 steps: 34 us
-// against 38 with two and 126 uncut; 48 tiles x 1021 bf16 steps 33, 36 and 78), two where one leaves a
-// third of the CUs idle (128 tiles x 1000 steps: 61 us against 67) or segments past 4096 steps, whose
-// end-state passes stop early (32 tiles x 65536 steps: 600 us against 640). At least 64 steps each,
-// none below 512, at most sqrt(L) of them: the output pass starts with a latency-bound chain over the
-// segments before its own, and a launch costs about 5 us.
-int64_t ps_segments(int64_t Bt, int64_t Dm, int64_t L) {
-    const int64_t pairs = ((Dm + 63) / 64) * Bt;
+// Time segments of scan_ps_kernel for Bt x Dm channels; drop: end-state passes stop early (ps_drop). At most
+// 128 (batch, 64-channel) tiles leave half of the 256 CUs idle, and cutting the sequence costs a second,
+// cheaper pass over it (1.75 times the work at most): worth it from there. One block per CU measured best (24
+// tiles x 2048 steps: 34 us against 38 with two and 126 uncut; 48 tiles x 1021 bf16 steps 33, 36 and 78), two
+// where one leaves a third of the CUs idle (128 tiles x 1000 steps: 61 us against 67), for segments past 4096
+// steps, whose end-state passes stop early (32 tiles x 65536 steps: 600 us against 640), and for long
+// sequences of 8 tiles and more whose passes do not (32 tiles x 65536 886 us against 1057, 24 x 8192 96
+// against 112; with 2 tiles the longer chain costs more, 125 against 110). At least 64
+// steps each, none below 512, at most sqrt(L) of them: the output pass starts with a latency-bound chain over the
+// segments before its own, and a launch costs about 5 us. More than half a tile per CU: two or three segments,
+// two blocks per CU, where the end-state pass stops early, from 8192 steps (fp32, uncut against cut: 129 tiles x
+// 8192 485 us and 393, x 16000 943 and 669; 192 x 8192 494 and 496, x 16000 965 and 900; 224 x 8192 568 and 512;
+// but 192 x 6000 364 and 383). Where it walks whole segments those sizes stay uncut.
+int64_t ps_segments(int64_t Bt, int64_t Dm, int64_t L, bool drop) {
+    const int64_t pairs = ((Dm + 63) / 64) * Bt, cus = device_cus();
     if (g_scan_segments > 0) return g_scan_segments;
-    if (pairs > 128 || L < 512) return 1;
-    int64_t nseg = 256 / pairs;
-    if (pairs > 85 || L > 4096 * nseg) nseg = 512 / pairs;
+    if (pairs >= cus || L < 512) return 1;
+    if (pairs > cus / 2) return drop && L >= 8192 ? 2 * cus / pairs : 1;
+    int64_t nseg = cus / pairs;
+    if (pairs > cus / 3 || (drop ? L > 4096 * nseg : L >= 8192 && pairs >= 8)) nseg = 2 * cus / pairs;
     if (nseg > L / 64) nseg = L / 64;
     while (nseg > 1 && nseg * nseg > L) --nseg;
     return nseg;
@@ -1788,8 +1794,8 @@ size_t ps_seg_bytes(int64_t Bt, int64_t Dm, int64_t nseg) {
     if (nseg <= 1) return 0;
     return (size_t)(nseg - 1) * 2 * Bt * ((Dm + 63) / 64) * 64 * 16 * sizeof(float);
 }
-size_t ps_workspace_bytes(int64_t Bt, int64_t Dm, int64_t L) {
-    return ps_seg_bytes(Bt, Dm, ps_seg_count(L, ps_seg_len(L, ps_segments(Bt, Dm, L))));
+size_t ps_workspace_bytes(int64_t Bt, int64_t Dm, int64_t L, bool drop) {
+    return ps_seg_bytes(Bt, Dm, ps_seg_count(L, ps_seg_len(L, ps_segments(Bt, Dm, L, drop))));
 }
 // Whether rows take the wave kernels' 16-byte accesses.
 bool tile_ok(const ScanArgs& a) {
@@ -1803,9 +1809,8 @@ size_t wave_workspace_bytes(const ScanArgs& a, size_t es);
 // of each segment's 4096. Shorter segments hardly reach that decay. All others walk whole segments, so that
 // a NaN, an infinity or an outlier reaches everything after it.
 constexpr int64_t kDropSteps = 4096;
-template <typename T>
-bool ps_drop(const ScanArgs& a) {
-    return a.L >= kDropSteps && !a.ws_may_be_short && wave_workspace_bytes(a, sizeof(T)) > 0;
+bool ps_drop(const ScanArgs& a, size_t es) {
+    return a.L >= kDropSteps && !a.ws_may_be_short && wave_workspace_bytes(a, es) > 0;
 }
 // scan_ps_kernel's sizes: a segment's byte offsets, a few chunks of read-ahead included, below 2^31, in the
 // rows of u, delta, z and out (Dm wide) and in those of B and C (16 wide).
@@ -1818,9 +1823,10 @@ template <typename T, bool HAS_Z, bool SP, int DTPK>
 int launch_ps(const ScanArgs& a, const uint16_t* dtlo, const uint16_t* wdt) {
     const int64_t ntiles = (a.Dm + 63) / 64;
     int64_t nseg = 1;
+    const bool drop = ps_drop(a, sizeof(T));
     if (a.ws) {
-        nseg = ps_segments(a.Bt, a.Dm, a.L);
-        const size_t need = ps_workspace_bytes(a.Bt, a.Dm, a.L);
+        nseg = ps_segments(a.Bt, a.Dm, a.L, drop);
+        const size_t need = ps_workspace_bytes(a.Bt, a.Dm, a.L, drop);
         const size_t least = a.ws_may_be_short ? 0 : wave_workspace_bytes(a, sizeof(T));
         HX_REQUIRE(least == 0 || (a.ws_bytes >= least && aligned(a.ws, 16)), HX_ERR_INVALID_INPUT,
                    "selective scan: workspace of %zu bytes (16-byte aligned) needed, %zu given "
@@ -1837,7 +1843,7 @@ int launch_ps(const ScanArgs& a, const uint16_t* dtlo, const uint16_t* wdt) {
     float4* hend = (float4*)a.ws;
     float4* decay = hend + (nseg - 1) * a.Bt * ntiles * 256;
     const PsArgs pa{a.L, a.Dm, (int)ntiles, (int)a.Bt, (int)nseg, (int)seg_len,
-                    ps_drop<T>(a), a.A, a.D, a.dt_bias,
+                    drop, a.A, a.D, a.dt_bias,
                     a.init_state, a.last_state, hend, decay, dtlo, wdt};
     if (nseg > 1) {
         hipLaunchKernelGGL((scan_ps_kernel<T, false, SP, true, DTPK>), dim3((unsigned)(ntiles * a.Bt * (nseg - 1))),
@@ -2055,7 +2061,7 @@ int run_scan(const ScanArgs& a) {
         // ones (8 x 2048 x 1536: 128 us against 135), unless the sequence is cut; sizes past the paired kernel's
         // offsets take the wave kernels where their float4 access is legal
         if (ps_ok(a.Bt, a.Dm, a.L, es)) {
-            const bool cut = a.ws && ps_segments(a.Bt, a.Dm, a.L) > 1;
+            const bool cut = a.ws && ps_segments(a.Bt, a.Dm, a.L, ps_drop(a, es)) > 1;
             if constexpr (std::is_same<T, float>::value)
                 if (!cut && tiles && ws2_ok<T>(a) && a.Bt * ((a.Dm + 47) / 48) <= device_cus())
                     return dispatch_ws<T, 3, true>(a);
@@ -2102,7 +2108,7 @@ size_t scan_workspace_bytes(const ScanArgs& a, size_t es) {
     if (a.N != 16 || a.L <= 0 || a.Bt <= 0 || a.Dm <= 0) return 0;
     if (v != 0 && v != 40 && v != 42) return 0;  // generic, fast and warp-specialised: none
     const size_t wave = wave_workspace_bytes(a, es);
-    const size_t ps = v == 0 && ps_ok(a.Bt, a.Dm, a.L, es) ? ps_workspace_bytes(a.Bt, a.Dm, a.L) : 0;
+    const size_t ps = v == 0 && ps_ok(a.Bt, a.Dm, a.L, es) ? ps_workspace_bytes(a.Bt, a.Dm, a.L, ps_drop(a, es)) : 0;
     return ps > wave ? ps : wave;
 }
 

@@ -555,3 +555,31 @@ def test_scan_short_workspace_of_rows_that_no_kernel_needed_it_for(dev, dim, off
         ssm.set_scan_segments(0)
     torch.cuda.synchronize()
     assert rel_err(out.cpu().numpy(), r64) <= TOL_F32
+
+
+@pytest.mark.parametrize("tiles,L,segments", [(129, 8191, 1), (129, 8192, 3), (171, 8192, 2), (255, 8200, 2), (256, 8192, 1)])
+def test_scan_segments_between_half_and_one_tile_per_cu(dev, tiles, L, segments):
+    """From 8192 steps sequences of more than half a (batch, 64-channel) tile per CU are cut as well: the bits of that
+    many forced segments, within rounding of the uncut scan. Dims that are no multiple of 4 stay uncut there."""
+    dim = tiles * 64
+    g = torch.Generator(device=dev).manual_seed(tiles + L)
+    n = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    x = dict(u=n(1, L, dim), delta=n(1, L, dim) * 0.5 - 4.0, B=n(1, L, 16), C=n(1, L, 16), z=n(1, L, dim))
+    x = {k: v.bfloat16() for k, v in x.items()}
+    A, D = -torch.arange(1.0, 17.0, device=dev).repeat(dim, 1), n(dim)
+
+    def run(d, nseg):
+        ssm.set_scan_segments(nseg)
+        try:
+            part = {k: v if v.shape[2] == 16 else v[..., :d].contiguous() for k, v in x.items()}
+            return ssm.selective_scan_fwd(**part, A=A[:d].contiguous(), D=D[:d].contiguous(), return_last_state=True)
+        finally:
+            ssm.set_scan_segments(0)
+
+    (auto, last), (forced, flast), (whole, wlast) = run(dim, 0), run(dim, segments), run(dim, 1)
+    assert torch.equal(auto, forced) and torch.equal(last, flast)
+    assert torch.equal(auto, whole) == (segments == 1)
+    assert norm_err(last.cpu(), wlast.cpu()) <= 4 * (3 * L) ** 0.5 * 2.0 ** -24
+    assert norm_err(auto.float().cpu(), whole.float().cpu()) <= 2.0 ** -8
+    if segments > 1:
+        assert torch.equal(run(dim - 1, 0)[0], run(dim - 1, 1)[0])
