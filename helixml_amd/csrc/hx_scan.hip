@@ -1819,6 +1819,16 @@ bool ps_ok(int64_t Bt, int64_t Dm, int64_t L, size_t es) {
     return L < (1LL << 30) && (L + 96) * row < (1LL << 31) && Bt * ((Dm + 63) / 64) <= 0x7fffffff;
 }
 
+// Many short sequences: each of scan_ps_kernel's blocks, two to a CU, reads three chunks ahead before its first
+// step, which a few steps do not pay for; the wave kernels keep more blocks in flight. us, paired against wave
+// kernel (the same bits): 4096 tiles x 1 step 33 and 25, x 32 45 and 40, x 96 bf16 102 and 99, x 128 128 and 130;
+// 1024 tiles x 16 10.8 and 9.5, x 48 18.7 and 18.0, x 64 21.5 and 22.2; with the fused dt projection (rank 128)
+// 4096 tiles x 16 58 and 41, x 64 95 and 85. At 512 tiles they are level.
+bool ps_brief(int64_t Bt, int64_t Dm, int64_t L) {
+    const int64_t tiles = Bt * ((Dm + 63) / 64), cus = device_cus();
+    return tiles >= 4 * cus && L <= (tiles >= 8 * cus ? 96 : 48);
+}
+
 template <typename T, bool HAS_Z, bool SP, int DTPK>
 int launch_ps(const ScanArgs& a, const uint16_t* dtlo, const uint16_t* wdt) {
     const int64_t ntiles = (a.Dm + 63) / 64;
@@ -2058,9 +2068,11 @@ int run_scan(const ScanArgs& a) {
     if (v == 0) {
         // auto: scan_ps_kernel; fp32 that fits one block per CU of the split-state warp-specialised
         // kernel, whose 48-channel blocks spread such a size over a third more CUs than 64-channel
-        // ones (8 x 2048 x 1536: 128 us against 135), unless the sequence is cut; sizes past the paired kernel's
-        // offsets take the wave kernels where their float4 access is legal
-        if (ps_ok(a.Bt, a.Dm, a.L, es)) {
+        // ones (8 x 2048 x 1536: 128 us against 135), unless the sequence is cut; many short sequences (ps_brief)
+        // and sizes past the paired kernel's offsets take the wave kernels where their float4 access is legal, and
+        // otherwise the fast kernel, which leads for one chunk (1536 tiles x 16 steps 11.5 us against 15, x 32 20
+        // against 19)
+        if (ps_ok(a.Bt, a.Dm, a.L, es) && !(ps_brief(a.Bt, a.Dm, a.L) && (tiles || a.L <= 16))) {
             const bool cut = a.ws && ps_segments(a.Bt, a.Dm, a.L, ps_drop(a, es)) > 1;
             if constexpr (std::is_same<T, float>::value)
                 if (!cut && tiles && ws2_ok<T>(a) && a.Bt * ((a.Dm + 47) / 48) <= device_cus())
@@ -2195,7 +2207,7 @@ int scan_fwd_dtproj(int64_t batch, int64_t seqlen, int64_t dim, const uint16_t* 
     HX_REQUIRE(aligned(u, 16) && aligned(z, 16) && aligned(out, 16) && aligned(dtlo, 16) && aligned(w_dt, 16) &&
                    aligned(B, 32) && aligned(C, 32) && (!D || aligned(D, 16)) && (!dt_bias || aligned(dt_bias, 16)),
                HX_ERR_UNSUPPORTED, "selective scan with dt_proj: operands not 16-byte aligned");
-    if (ps_ok(batch, dim, seqlen, 2)) {
+    if (ps_ok(batch, dim, seqlen, 2) && !ps_brief(batch, dim, seqlen)) {
         const ScanArgs a{batch, seqlen, dim, 16, 1, u, nullptr, A, B, C, D, z, dt_bias, out, nullptr, last_state,
                          stream, ws, ws_bytes, true};
         switch (rank / 32) {

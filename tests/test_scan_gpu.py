@@ -370,6 +370,25 @@ def test_scan_dtproj_matches_separate_steps(dev, bt, L, dim, r):
     assert e_sep <= 4e-3 and e_ref <= 1e-2, (e_sep, e_ref)
 
 
+@pytest.mark.parametrize("bt,L,dim,r", [(1024, 16, 64, 32), (1024, 48, 60, 128), (2048, 96, 64, 64), (1024, 49, 64, 96)])
+def test_scan_dtproj_many_short_sequences(dev, bt, L, dim, r):
+    """Too many short sequences for the paired kernel's read-ahead take the wave kernel, with the same bits as a few
+    of them alone."""
+    g = torch.Generator(device=dev).manual_seed(L + r)
+    rnd = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
+    x = [rnd(bt, L, w).bfloat16() for w in (dim, r, 16, 16, dim)]  # u, dt_lo, B, C, z
+    w_dt, D, dt_bias = (rnd(dim, r) / r ** 0.5).bfloat16(), rnd(dim), rnd(dim) * 0.5 - 4.0
+    A = -torch.arange(1.0, 17.0, device=dev).repeat(dim, 1)
+
+    def run(u, dt_lo, B, C, z):
+        return ssm.selective_scan_dtproj_fwd(u, dt_lo, w_dt, A, B, C, D, z, dt_bias, return_last_state=True)
+
+    out, last = run(*x)
+    for b in (0, bt - 4):
+        few, flast = run(*[t[b:b + 4].contiguous() for t in x])
+        assert torch.equal(out[b:b + 4], few) and torch.equal(last[b:b + 4], flast)
+
+
 def test_scan_dtproj_errors_and_empty(dev):
     """hx_selective_scan_dtproj_fwd takes dt_rank 32, 64, 96 or 128 and dim % 4 == 0 (else
     UnsupportedOperation, nothing launched), needs every operand but D, dt_bias and last_state
@@ -423,6 +442,27 @@ def test_scan_paired_kernel_matches_wave_kernel_bitwise(dev, bt, L, dim, with_z)
         ssm.set_scan_segments(0)
     assert np.array_equal(auto[0], wave[0])
     assert np.array_equal(auto[1], wave[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("bt,L,dim", [(1023, 48, 60), (1024, 1, 64), (1024, 48, 60), (1024, 49, 64), (2048, 96, 4),
+                                      (2048, 97, 8), (1024, 16, 62), (1024, 17, 62)])
+def test_scan_many_short_sequences(dev, bt, L, dim, dtype):
+    """Either side of the sizes whose short sequences are too many for the paired kernel's read-ahead: rows of
+    16-byte pieces give the wave kernel's bits whichever kernel takes them, the others agree with the float64
+    restatement, with an initial state and the final state."""
+    x = scan_inputs(bt, L, dim, 16, seed=L * 7 + dim, with_bias=True)
+    if dtype == torch.bfloat16:
+        x = {k: (bf16_round(v) if k not in ("A", "D", "dt_bias") else v) for k, v in x.items()}
+    init = (np.random.default_rng(L).standard_normal((bt, dim, 16)) * 0.5).astype(np.float32)
+    auto = run_gpu(x, dev, dtype=dtype, init_state=init, last=True)
+    if dim % 4 == 0:
+        ssm.set_scan_variant(42)
+        wave = run_gpu(x, dev, dtype=dtype, init_state=init, last=True)
+        assert np.array_equal(auto[0], wave[0]) and np.array_equal(auto[1], wave[1])
+    r64, rlast64 = oracle.numpy_selective_scan(**x, init_state=init)
+    assert norm_err(auto[1], rlast64) <= 4 * (3 * L) ** 0.5 * 2.0 ** -24
+    assert norm_err(auto[0], r64) <= (2.0 ** -8 if dtype == torch.bfloat16 else TOL_F32)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
