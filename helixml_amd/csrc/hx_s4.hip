@@ -1291,7 +1291,10 @@ extern "C" int hx_s4_ref_fwd(int64_t d_model, int64_t dstate, int64_t seqlen, fl
             hipLaunchKernelGGL(s4_input_proj_kernel<4>, g1, dim3(256), 0, s, d_model, seqlen, dstate,
                                Np, x, BdT, H);
     }
-    if (dstate <= 16 && seqlen <= kFuseT) {
+    // every block repeats the chain: worth it up to kPlMaxM channels, one round of blocks (2048 x 512 78 us
+    // against 181); past that the rounds add up (8192 x 512 723 against 679) except for short chains (2049 x 64
+    // 172 against 178, 8192 x 64 level)
+    if (dstate <= 16 && seqlen <= kFuseT && (d_model <= kPlMaxM || seqlen <= 64)) {
         hipLaunchKernelGGL(s4_scan_output_kernel, dim3((unsigned)((d_model + kTileM - 1) / kTileM),
                                                        (unsigned)((seqlen + kFuseTile - 1) / kFuseTile)),
                            dim3(256), 0, s, d_model, seqlen, (int)dstate, x, a, H, C, D, gate, y);

@@ -114,11 +114,13 @@ def test_s4_ref_bit_exact_paths(dev, M, N, L, offset):
 @pytest.mark.parametrize("M,N,L,offset", [
     (1, 1, 1, 0), (15, 5, 512, 0), (17, 16, 513, 1), (64, 16, 511, 0), (130, 7, 65, 1),  # 4-state blocks, edges
     (2048, 4, 70, 0), (2049, 4, 70, 0),      # the most rows whose B fits beside its ring, and one more
+    (2048, 16, 512, 0), (2049, 16, 512, 0),  # the most channels of the fused recurrence and output, and one more,
+    (2049, 16, 64, 0), (2049, 16, 65, 0),    # which it takes up to 64 steps
     (64, 16, 4097, 0), (70, 16, 4200, 0), (37, 16, 4200, 1), (19, 33, 2100, 0),  # more waves: the ring kernel
 ])
 def test_s4_ref_bit_exact_projection_choice(dev, M, N, L, offset):
     """Both sides of the choice of projection kernel and of the fused recurrence and output (at most 512
-    steps and 16 states), x aligned and not."""
+    steps and 16 states, 64 steps past 2048 channels), x aligned and not."""
     test_s4_ref_bit_exact_paths(dev, M, N, L, offset)
 
 
