@@ -1345,27 +1345,6 @@ namespace {
 thread_local int g_s4d_path = 0;  // per calling thread (hx_set_s4d_path)
 thread_local int g_s4d_segments = 0;  // per calling thread (hx_set_s4d_segments)
 
-// Time segments of the S4D wave path, 16-step aligned: two blocks per CU (1 x 65536 x 2048: 474 us with
-// 16, 632 with 8, 476 with 32), at least 64 steps each and at most sqrt(L) / 2 of them, as each one chains
-// those before it (1 x 16384 x 256: 60 us with 64, 78 with 32, 88 with 128). Segments of at least 512
-// steps, the rule before, left short sequences of few channels on a handful of blocks: 1 x 4096 x 64
-// 71 us with 8, 35 with 32; 2 x 2000 x 300 104 with 2, 30 with 25; 3 x 1000 x 2048 76 with 1, 48 with 5. Below
-// 320 steps the second launch costs what the shorter chain saves (1 x 256 x 128: 23 us with 1, 22 with 4).
-// Returns the segment count and sets seg_len.
-int64_t s4d_segments(int64_t Bt, int64_t L, int64_t Dm, int64_t* seg_len_out) {
-    const int64_t pairs = (int64_t)((Dm + 63) / 64) * Bt;
-    int64_t nseg = g_s4d_segments;
-    if (nseg <= 0) {
-        nseg = (512 + pairs - 1) / pairs;
-        const int64_t cap = L >= 320 ? L / 64 : 1;
-        nseg = nseg < cap ? nseg : cap;
-        while (nseg > 1 && 4 * nseg * nseg > L) --nseg;
-    }
-    int64_t seg_len = (L + nseg - 1) / nseg;
-    seg_len = (seg_len + 15) / 16 * 16;
-    *seg_len_out = seg_len;
-    return (L + seg_len - 1) / seg_len;
-}
 // Segments of at least 512 steps, two waves per SIMD: end states that decay inside such a segment start
 // late in it, and their room (end and entry states) is what a given workspace must have. Sequences that
 // these leave whole need no workspace, and their end states leave nothing out.
@@ -1380,11 +1359,38 @@ int64_t s4d_long_segments(int64_t Bt, int64_t L, int64_t Dm) {
     const int64_t seg_len = ((L + nseg - 1) / nseg + 15) / 16 * 16;
     return (L + seg_len - 1) / seg_len;
 }
-bool s4d_wave_ok(int64_t dstate) { return dstate == 16 && g_s4d_path != 1; }
 // Whether rows take 16-byte accesses. The others, with 4-byte ones, against one thread a channel over the
 // whole sequence, which took them before: 1 x 100 x 65 23 us against 49, 2 x 2000 x 301 34 against 819,
 // 1 x 65536 x 2047 0.91 ms against 44.6. They need no workspace and leave nothing out.
 bool s4d_vec_ok(int64_t dim, const float* x, const float* y) { return dim % 4 == 0 && aligned(x, 16) && aligned(y, 16); }
+
+// Time segments of the S4D wave path, 16-step aligned; whole: end states leave nothing out, so cutting costs a
+// second pass over the sequence. Two blocks per CU (1 x 65536 x 2048: 474 us with
+// 16, 632 with 8, 476 with 32), at least 64 steps each and at most sqrt(L) / 2 of them, as each one chains
+// those before it (1 x 16384 x 256: 60 us with 64, 78 with 32, 88 with 128). Segments of at least 512
+// steps, the rule before, left short sequences of few channels on a handful of blocks: 1 x 4096 x 64
+// 71 us with 8, 35 with 32; 2 x 2000 x 300 104 with 2, 30 with 25; 3 x 1000 x 2048 76 with 1, 48 with 5. Below
+// 320 steps the second launch costs what the shorter chain saves (1 x 256 x 128: 23 us with 1, 22 with 4). The more
+// (batch, 64-channel) tiles, the less a second whole pass gains: 128 tiles x 400 steps 33.5 us whole, 34.7 cut, x
+// 500 41 and 36; 192 x 800 62 and 65, x 1400 104 and 98; 256 x 1000 77 and 82, from there on in every length
+// (400, 4-byte accesses, x 2000 223 and 285).
+// Returns the segment count and sets seg_len.
+int64_t s4d_segments(int64_t Bt, int64_t L, int64_t Dm, bool whole, int64_t* seg_len_out) {
+    const int64_t pairs = (int64_t)((Dm + 63) / 64) * Bt;
+    int64_t nseg = g_s4d_segments;
+    if (nseg <= 0) {
+        const bool uncut = L < 320 || (whole && (pairs >= 256 || (L < 1024 && (pairs >= 192 || 4 * L < 15 * pairs))));
+        nseg = (512 + pairs - 1) / pairs;
+        const int64_t cap = uncut ? 1 : L / 64;
+        nseg = nseg < cap ? nseg : cap;
+        while (nseg > 1 && 4 * nseg * nseg > L) --nseg;
+    }
+    int64_t seg_len = (L + nseg - 1) / nseg;
+    seg_len = (seg_len + 15) / 16 * 16;
+    *seg_len_out = seg_len;
+    return (L + seg_len - 1) / seg_len;
+}
+bool s4d_wave_ok(int64_t dstate) { return dstate == 16 && g_s4d_path != 1; }
 // Bytes of one segment's end states, [B][D][16] complex.
 size_t s4d_seg_bytes(int64_t Bt, int64_t Dm) { return (size_t)Bt * Dm * 16 * 2 * sizeof(float); }
 size_t s4d_least_bytes(int64_t Bt, int64_t L, int64_t Dm) {
@@ -1393,8 +1399,10 @@ size_t s4d_least_bytes(int64_t Bt, int64_t L, int64_t Dm) {
 }
 size_t s4d_ws_bytes(int64_t Bt, int64_t L, int64_t Dm) {
     int64_t seg_len = 0;
-    const size_t need = (s4d_segments(Bt, L, Dm, &seg_len) - 1) * s4d_seg_bytes(Bt, Dm);
-    const size_t least = Dm % 4 == 0 ? s4d_least_bytes(Bt, L, Dm) : 0;
+    const bool vec = Dm % 4 == 0;  // pointers assumed aligned
+    const bool whole = !vec || s4d_long_segments(Bt, L, Dm) == 1;
+    const size_t need = (s4d_segments(Bt, L, Dm, whole, &seg_len) - 1) * s4d_seg_bytes(Bt, Dm);
+    const size_t least = vec ? s4d_least_bytes(Bt, L, Dm) : 0;
     return need > least ? need : least;
 }
 
@@ -1404,16 +1412,17 @@ int launch_s4d_wave(int64_t Bt, int64_t L, int64_t Dm, const float* x, const flo
                     float* scratch, size_t scratch_bytes, hipStream_t s) {
     const int ntiles = (int)((Dm + 63) / 64);
     const int64_t pairs = (int64_t)ntiles * Bt;
+    const bool vec = s4d_vec_ok(Dm, x, y);
+    const bool whole = !vec || s4d_long_segments(Bt, L, Dm) == 1;
     int64_t seg_len = L;
-    int64_t nseg = s4d_segments(Bt, L, Dm, &seg_len);
+    int64_t nseg = s4d_segments(Bt, L, Dm, whole, &seg_len);
     const int64_t room = scratch && aligned(scratch, 16) ? 1 + (int64_t)(scratch_bytes / s4d_seg_bytes(Bt, Dm)) : 1;
     if (nseg > room) {  // as many as fit
         seg_len = ((L + room - 1) / room + 15) / 16 * 16;
         nseg = (L + seg_len - 1) / seg_len;
     }
     HX_REQUIRE(pairs * nseg <= 0x7fffffff, HX_ERR_UNSUPPORTED, "s4d_complex: grid too large");
-    const bool vec = s4d_vec_ok(Dm, x, y);
-    const S4dSeg sg{seg_len, (int)nseg, !vec || s4d_long_segments(Bt, L, Dm) == 1, scratch};
+    const S4dSeg sg{seg_len, (int)nseg, whole, scratch};
     auto run = [&](auto kernel, int64_t segs) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)(pairs * segs)), dim3(256), 0, s, L, Dm, ntiles, Bt, x, dt,
                            a_re, a_im, B_re, B_im, C_re, C_im, D, y, sg);

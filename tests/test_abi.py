@@ -88,6 +88,16 @@ def test_gemm_without_its_lds_falls_through(M, N, K):
     assert rc == _ffi.BackendError.status, _ffi.last_error()
 
 
+@pytest.mark.parametrize("dim,L,cut", [
+    (128 * 64, 479, False), (128 * 64, 480, True), (96 * 64 - 3, 359, False), (96 * 64 - 3, 360, True), (1, 319, False), (1, 320, True),
+    (191 * 64, 717, True), (192 * 64, 1023, False), (192 * 64 - 1, 1024, True), (256 * 64 - 1, 4096, False), (256 * 64, 1024, True)])
+def test_s4d_segments_where_a_second_pass_pays(dim, L, cut):
+    """Sequences whose end states leave nothing out (below 1024 steps, or dims that are no multiple of 4) are cut, which
+    takes a workspace, only where the second pass is repaid: with tiles of 64 channels, from 15/4 steps a tile, none from
+    192 below 1024 steps and from 256 at any length."""
+    assert (_ffi.lib().hx_s4d_workspace_size(1, L, dim, 16) > 0) == cut
+
+
 def test_s4_ref_rejects():
     L = _ffi.lib()
     assert L.hx_s4_ref_fwd(4, 0, 4, 0.1, *([None] * 7), None, 0, None) == _ffi.UnsupportedOperation.status
