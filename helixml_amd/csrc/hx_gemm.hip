@@ -490,87 +490,123 @@ __device__ inline void store_slab_fast(char* __restrict__ yb, int64_t ldb, const
     }
 }
 
-// Writes a wave's staged nrows x 64 fp32 tile (st, row stride 68) to the outputs: rows of 64
-// columns as 16-byte vectors (8 bf16 or 4 fp32 per lane) with bias, SiLU and accumulate; a
-// vector that would straddle a column split or the N edge falls back to element stores.
-__device__ inline void store_tile_rows(const GemmOut& o, const float* __restrict__ bias,
-                                       const float* st, int64_t M, int64_t N, int64_t row0,
-                                       int64_t col0, int lane, int nrows = 32) {
-        // rows of 64 columns: o.out_bf16 -> 8 lanes x 8 columns per row (8 rows per pass),
-        // fp32 -> 16 lanes x 4 columns per row (4 rows per pass)
-        const int vw = o.out_bf16 ? 8 : 4;
-        const int lpr = 64 / vw;             // lanes per row
-        const int rpp = 64 / lpr;            // rows per pass
-        const int rl = lane / lpr, cl = (lane % lpr) * vw;
-        for (int rr = rl; rr < nrows; rr += rpp) {
-            const int64_t row = row0 + rr;
-            const int64_t col = col0 + cl;
-            if (row >= M || col >= N) continue;
-            float v[8];
+// Writes the first `rows` rows and `cols` columns (whole vectors) of a staged ROWS x 64 fp32 slab (st, row stride 68)
+// that lies inside one output with 16-byte aligned rows: 16-byte vectors, with bias, SiLU and accumulate. All reads of
+// the slab and of the existing outputs go out before the first store. yb: the slab's first output element, ldb:
+// row pitch in bytes.
+template <bool BF16, int ROWS>
+__device__ inline void store_slab_rows(const GemmOut& o, const float* __restrict__ bias, const float* st,
+                                       char* __restrict__ yb, int64_t ldb, int rows, int cols, int64_t col0, int lane) {
+    using G = SlabGeom<BF16, ROWS>;
+    typedef float f32v4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(1))) slab_u32v4 g_u32v4;
+    typedef __attribute__((address_space(3))) const f32v4 l_f32v4;
+    constexpr int NP = G::NP, VW = G::VW;
+    const int rl = lane / G::LPR, cl = (lane % G::LPR) * VW;
+    if (cl >= cols) return;
+    char* yp = yb + cl * (BF16 ? 2 : 4);
+    f32v4 v[NP][VW / 4];
+    slab_u32v4 old[NP];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                if (q < vw) {
-                    float x = st[rr * 68 + cl + q];
-                    if (bias && col + q < N) x += bias[col + q];
-                    if (o.act & 1) x = silu(x);
-                    v[q] = x;
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int h = 0; h < VW / 4; ++h) v[p][h] = ((l_f32v4*)(st + (p * G::RPP + rl) * 68 + cl))[h];
+    if (o.act & 2) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            const int r = p * G::RPP + rl;
+            old[p] = *(g_u32v4*)(yp + (r < rows ? r : rows - 1) * ldb);
+        }
+    }
+    if (bias) {
+#pragma unroll
+        for (int q = 0; q < VW; ++q) {
+            const float bq = bias[col0 + cl + q];
+#pragma unroll
+            for (int p = 0; p < NP; ++p) v[p][q / 4][q % 4] += bq;
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int r = p * G::RPP + rl;
+        float f[VW];
+#pragma unroll
+        for (int q = 0; q < VW; ++q) f[q] = (o.act & 1) ? silu(v[p][q / 4][q % 4]) : v[p][q / 4][q % 4];
+        slab_u32v4 w;
+        if constexpr (BF16) {
+            if (o.act & 2) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    f[2 * k] += __uint_as_float(old[p][k] << 16);
+                    f[2 * k + 1] += __uint_as_float(old[p][k] & 0xffff0000u);
                 }
             }
-            int seg = 0;
-            int64_t cc = col;
-            if (col >= o.split2) { seg = 2; cc = col - o.split2; }
-            else if (col >= o.split1) { seg = 1; cc = col - o.split1; }
-            const int64_t seg_end = seg == 0 ? o.split1 : seg == 1 ? o.split2 : N;
-            const int64_t off = row * o.ldp(seg) + cc;
-            const bool whole = col + vw <= seg_end &&
-                               ((uintptr_t)((char*)o.yp(seg) + off * (o.out_bf16 ? 2 : 4)) & 15) == 0;
-            if (whole) {
-                if (o.out_bf16) {
-                    uint16_t* yp = (uint16_t*)o.yp(seg) + off;
-                    if (o.act & 2) {
-                        const uint4 old = *reinterpret_cast<const uint4*>(yp);
-                        const uint32_t ow[4] = {old.x, old.y, old.z, old.w};
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            v[2 * q] += __uint_as_float(ow[q] << 16);
-                            v[2 * q + 1] += __uint_as_float(ow[q] & 0xffff0000u);
-                        }
-                    }
-                    uint32_t wv[4];
+            for (int k = 0; k < 4; ++k) w[k] = pack_bf16x2(f[2 * k], f[2 * k + 1]);
+        } else {
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        wv[q] = pack_bf16x2(v[2 * q], v[2 * q + 1]);
-                    *reinterpret_cast<uint4*>(yp) = make_uint4(wv[0], wv[1], wv[2], wv[3]);
-                } else {
-                    float* yp = (float*)o.yp(seg) + off;
-                    if (o.act & 2) {
-                        const float4 old = *reinterpret_cast<const float4*>(yp);
-                        v[0] += old.x; v[1] += old.y; v[2] += old.z; v[3] += old.w;
-                    }
-                    *reinterpret_cast<float4*>(yp) = make_float4(v[0], v[1], v[2], v[3]);
-                }
-            } else {
-                for (int q = 0; q < vw; ++q) {
-                    const int64_t cq = col + q;
-                    if (cq >= N) break;
-                    int sq = 0;
-                    int64_t ccq = cq;
-                    if (cq >= o.split2) { sq = 2; ccq = cq - o.split2; }
-                    else if (cq >= o.split1) { sq = 1; ccq = cq - o.split1; }
-                    const int64_t oq = row * o.ldp(sq) + ccq;
-                    float x = v[q];
-                    if (o.out_bf16) {
-                        uint16_t* yp = (uint16_t*)o.yp(sq) + oq;
-                        if (o.act & 2) x += Storage<uint16_t>::load(yp);
-                        Storage<uint16_t>::store(yp, x);
-                    } else {
-                        float* yp = (float*)o.yp(sq) + oq;
-                        if (o.act & 2) x += *yp;
-                        *yp = x;
-                    }
-                }
+            for (int k = 0; k < 4; ++k) w[k] = __float_as_uint((o.act & 2) ? f[k] + __uint_as_float(old[p][k]) : f[k]);
+        }
+        if (r < rows) *(g_u32v4*)(yp + r * ldb) = w;
+    }
+}
+
+// Writes a wave's staged ROWS x 64 fp32 tile (st, row stride 68) to the outputs, with bias, SiLU and accumulate; its
+// columns end at N. Whole 16-byte vectors inside one output: store_slab_rows. Otherwise (a column split or a ragged end
+// inside the tile, rows of another alignment) a lane owns a column and a row goes out as 64 neighbouring elements, eight rows at a time.
+// Bound by the stores' issue. A lane used to hold 8 (4 fp32) neighbouring columns on both paths and stored them one
+// by one here, each instruction touching 8 rows; 4000 x 2047 x 256 on 256 x 256 tiles took 95 us of it, 8192 x 3500
+// x 256 187.
+template <int ROWS = 32>
+__device__ inline void store_tile_rows(const GemmOut& o, const float* __restrict__ bias, const float* st, int64_t M,
+                                       int64_t N, int64_t row0, int64_t col0, int lane) {
+    if (row0 >= M || col0 >= N) return;  // uniform
+    const int rows = M - row0 < ROWS ? (int)(M - row0) : ROWS, cols = N - col0 < 64 ? (int)(N - col0) : 64;
+    const int es = o.out_bf16 ? 2 : 4;
+    {
+        const int seg = col0 >= o.split2 ? 2 : col0 >= o.split1 ? 1 : 0;
+        const int64_t seg_lo = seg == 2 ? o.split2 : seg == 1 ? o.split1 : 0;
+        const int64_t seg_end = seg == 0 ? o.split1 : seg == 1 ? o.split2 : N;
+        const int64_t ldb = o.ldp(seg) * es;
+        char* yb = (char*)o.yp(seg) + row0 * ldb + (col0 - seg_lo) * es;
+        if (col0 + cols <= seg_end && (((uintptr_t)yb | (uint64_t)ldb | (uint64_t)(cols * es)) & 15) == 0) {
+            if (o.out_bf16) store_slab_rows<true, ROWS>(o, bias, st, yb, ldb, rows, cols, col0, lane);
+            else store_slab_rows<false, ROWS>(o, bias, st, yb, ldb, rows, cols, col0, lane);
+            return;
+        }
+    }
+    if (lane >= cols) return;
+    const int64_t col = col0 + lane;
+    const int seg = col >= o.split2 ? 2 : col >= o.split1 ? 1 : 0;
+    const int64_t seg_lo = seg == 2 ? o.split2 : seg == 1 ? o.split1 : 0;
+    const int64_t ldb = o.ldp(seg) * es;
+    char* yb = (char*)o.yp(seg) + row0 * ldb + (col - seg_lo) * es;
+    const float bv = bias ? bias[col] : 0.0f;
+    typedef __attribute__((address_space(1))) uint16_t g_u16;
+    typedef __attribute__((address_space(1))) float g_f32;
+    typedef __attribute__((address_space(3))) const float l_f32;
+    for (int r0 = 0; r0 < rows; r0 += 8) {
+        float v[8], old[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            v[q] = ((l_f32*)st)[(r0 + q) * 68 + lane];
+            if (o.act & 2) {
+                const char* p = yb + (r0 + q < rows ? r0 + q : rows - 1) * ldb;
+                old[q] = o.out_bf16 ? bf16_bits_to_f32(*(g_u16*)p) : *(g_f32*)p;
             }
         }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            if (r0 + q >= rows) break;  // uniform
+            float x = v[q];
+            if (bias) x += bv;
+            if (o.act & 1) x = silu(x);
+            if (o.act & 2) x += old[q];
+            char* p = yb + (r0 + q) * ldb;
+            if (o.out_bf16) *(g_u16*)p = Storage<uint16_t>::round(x);
+            else *(g_f32*)p = x;
+        }
+    }
 }
 
 // Tile order of the big-tile kernels (blocks = tiles, one or two per CU). Consecutive block ids
@@ -1391,25 +1427,24 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_d256p_kernel(int64_t M, int6
             sprev = o.out_bf16 ? 16 * SlabGeom<true, 16>::NP : 16 * SlabGeom<false, 16>::NP;
         } else {
             sprev = 0;
+            // a loop at run time, with one copy of the stores: sixteen copies hold more registers than there are
+#pragma unroll 1
+            for (int sl = 0; sl < 16; ++sl) {  // slab (a, h, jj) = (sl / 4, sl / 2 % 2, sl % 2)
+                StepLoop<16>::run([&](auto kc) __attribute__((always_inline)) {
+                    constexpr int k = decltype(kc)::value, a = k >> 2, h = (k >> 1) & 1, jj = k & 1;
+                    if (sl != k) return;
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
+                    for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-#pragma unroll
-                    for (int jj = 0; jj < 2; ++jj) {
-#pragma unroll
-                        for (int j = 0; j < 2; ++j)
-#pragma unroll
-                            for (int rr = 0; rr < 8; ++rr) {
-                                const int r = 8 * h + rr;
-                                const int row = 8 * ((r >> 2) - 2 * h) + 4 * (lane >> 5) + (r & 3);
-                                st[row * 68 + j * 32 + (lane & 31)] = acc[a][2 * jj + j][r];
-                            }
-                        __builtin_amdgcn_wave_barrier();
-                        store_tile_rows(o, bias, st, M, N, r0 + a * 32 + h * 16, c0 + jj * 64, lane, 16);
-                        __builtin_amdgcn_wave_barrier();
-                    }
-                }
+                        for (int rr = 0; rr < 8; ++rr) {
+                            const int r = 8 * h + rr;
+                            const int row = 8 * ((r >> 2) - 2 * h) + 4 * (lane >> 5) + (r & 3);
+                            st[row * 68 + j * 32 + (lane & 31)] = acc[a][2 * jj + j][r];
+                        }
+                });
+                __builtin_amdgcn_wave_barrier();
+                store_tile_rows<16>(o, bias, st, M, N, r0 + sl / 4 * 32 + sl / 2 % 2 * 16, c0 + sl % 2 * 64, lane);
+                __builtin_amdgcn_wave_barrier();
             }
         }
 #pragma unroll

@@ -392,3 +392,40 @@ def test_gemm_middle_sizes(dev, M, N, K):
         finally:
             ssm.set_gemm_kernel(0)
         assert torch.equal(same, torch.cat(outs, 1))
+
+
+@pytest.mark.parametrize("gemm_kernel", [0, 4, 5, 7, 8], indirect=True)
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,split,pad,act", [
+    (300, 250, 0, 0, 0), (257, 256, 0, 1, 0), (290, 136, 0, 3, 2),  # ragged N; rows of another alignment, accumulated into
+    (271, 255, 100, 0, 1), (321, 192, 64, 8, 3), (260, 72, 30, 2, 3), (513, 544, 31, 0, 2)])  # splits, SiLU
+def test_gemm_edge_stores(dev, gemm_kernel, out_dtype, M, N, split, pad, act):
+    """The tile kernels' guarded epilogue on both its paths, 16-byte vectors and single elements: ends and column
+    splits inside a 64-column slab, row pitches that are and are not multiples of 16 bytes, bias, SiLU (bit 0) and
+    accumulate (bit 1), and nothing written between or past the rows. Bars as in test_gemm_middle_sizes."""
+    from helixml_amd import _ffi
+    K = 192
+    g = torch.Generator(device=dev).manual_seed(M + N + act)
+    X = torch.randn(M, K, generator=g, device=dev).bfloat16()
+    W = (torch.randn(N, K, generator=g, device=dev) / K ** 0.5).bfloat16()
+    bias = torch.randn(N, generator=g, device=dev) if act & 1 else None
+    widths = [split, N - split] if split else [N]
+    bufs = [torch.randn(M + 1, w + pad, generator=g, device=dev).to(out_dtype) for w in widths]
+    before = [b.clone() for b in bufs]
+    p1 = bufs[1].data_ptr() if split else None
+    _ffi.call("hx_gemm_bf16", M, N, K, X.data_ptr(), K, W.data_ptr(), K, bias.data_ptr() if act & 1 else None, act,
+              _ffi.HX_F32 if out_dtype == torch.float32 else _ffi.HX_BF16, bufs[0].data_ptr(), widths[0] + pad,
+              split or N, p1, widths[-1] + pad, N, None, 0, torch.cuda.current_stream().cuda_stream)
+    ref = X.double() @ W.double().T
+    bound = (K + 2) * 2.0 ** -24 * (X.double().abs() @ W.double().abs().T)
+    if act & 1:
+        ref = ref + bias.double()
+        ref, bound = ref * torch.sigmoid(ref), 1.2 * bound + 1e-5
+    c = 0
+    for b, old, w in zip(bufs, before, widths):
+        want = ref[:, c:c + w] + (old[:M, :w].double() if act & 2 else 0)
+        tol = bound[:, c:c + w] + want.abs() * (2.0 ** -8 if out_dtype == torch.bfloat16 else 2.0 ** -23)
+        err = (b[:M, :w].double() - want).abs() - tol
+        assert bool((err <= 0).all()), float(err.max())
+        assert torch.equal(b[:, w:], old[:, w:]) and torch.equal(b[M], old[M])
+        c += w
