@@ -1613,8 +1613,8 @@ bool gemm_rmsnorm_small_ok(int64_t M, int64_t N, int64_t K, const float* X, int6
         return false;
     if (ldx % 4 != 0 || ldw % 8 != 0 || !aligned(X, 16) || !aligned(nw, 16) || !aligned(W, 16))
         return false;
-    // hx_gemm_bf16 takes the small-M kernel for these sizes (its other forms need K >= 1024 or
-    // at least 128 tiles of 128 x 128)
+    // sizes of the small-M kernel's range, fewer than 128 tiles of 128 x 128 (hx_gemm_bf16 takes the larger of
+    // them to its narrow kernel)
     if (((M + BM - 1) / BM) * ((N + BN - 1) / BN) >= 128 || (M + 31) / 32 > 65535) return false;
     return skinny_shape(M, N, K).spw <= 4;  // one round of at most 4 pieces per lane
 }
@@ -1706,33 +1706,65 @@ extern "C" int hx_gemm_bf16(int64_t M, int64_t N, int64_t K, const void* X, int6
         return launch_d256<64, 2>(M, N, K, X, ldx, W, ldw, bias, o, stream);
     if (vec && K > 0 && K % 32 == 0 && (g_gemm_kernel == 6 || (d256_auto && K % 64 != 0)) && d256_ok<32, 4>())
         return launch_d256<32, 4>(M, N, K, X, ldx, W, ldw, bias, o, stream);
-    // auto, too few 256 x 256 tiles for one per CU. From 112 of them that kernel still leads (4000 x 2048 x
-    // 512: 20 us against 26 with 64 x 128 tiles; at 96, 1999 x 3072 x 768, 31 against 26). Below, and where K
-    // is no multiple of 64, the narrow kernel's 64-row tiles over a grid of columns: 128 wide, or 64 where
-    // those leave CUs idle (777 x 1024 x 2048, 104 wide tiles: 18 us against 21). Against the kernels
-    // that took these before: 1999 x 768 x 1536 38 -> 18 us, 2867 x 1736 x 3472 133 -> 84, 48 x 2048 x 4096
-    // 76 -> 26. Same K-ascending 16-wide MFMA sums as the 256 x 256 kernel's, so a short batch that
-    // lands here matches a long one there. Short K and few outputs stay with the small-M kernel (1000 x
-    // 512 x 1024: 8.5 us against 10.5; level at 32-square tiles x K of 2^19: 500 x 2048 x 512), except from
-    // K = 2048 on, where its K split would give a prefix other bits than the whole.
-    const bool small_out = K < 2048 && ((M + 31) / 32) * ((N + 31) / 32) * K <= (1 << 19);
+    // auto, too few 256 x 256 tiles for one per CU (or K no multiple of 32). us in the order of the kernels named:
+    // * the 256 x 256 kernel still leads from 112 tiles (4096 x 2048 x 512: 15 against 19 on 64 x 128 tiles). Tiles
+    //   that are not stored whole cost its few waves a guarded epilogue: with more than 32 rows or columns of a
+    //   wave's 128 x 128 so, from K = 512 (4096 x 2000 x 128 17 and 11, x 512 23 and 19, 6000 x 1480 x 512 25 and
+    //   24, x 1024 33 and 40) or 160 tiles (30000 x 320 x 64 11 and 12), and with output rows of another alignment
+    //   from K = 1024 and 160 tiles (4000 x 3500 x 768 51 and 54, x 1024 57 and 65; 4000 x 2047 x 1024 53 and 39);
+    // * the 256 x 128 kernel, one block per CU: long K where its blocks make one nearly whole round (4100 x 1480 x
+    //   4096: 79 against 95 on 64 x 128 tiles, 4000 x 2047 x 4096 93 and 112), K >= 1024 for many rows of 129 to
+    //   255 columns (131072 x 200 x 2048 221 and 273), and one panel of 129 to 256 rows against a W that no cache
+    //   holds, which 64-row tiles read two to four times (200 x 16384 x 4096 78 and 125; 256 x 32768 x 4096
+    //   87, the 256 x 256 kernel 101);
+    // * else the narrow kernel's 64-row tiles over a grid of columns: 128 wide, or 64 where those leave CUs idle
+    //   (777 x 1024 x 2048, 104 wide tiles: 18 against 21). Against the kernels that took these before: 1999 x 768
+    //   x 1536 38 and 18, 2867 x 1736 x 3472 133 and 83, 48 x 2048 x 4096 76 and 26. Same K-ascending 16-wide
+    //   MFMA sums as the 256 x 256 kernel's, so a short batch that lands here matches a long one there;
+    // * K no multiple of 64 with many tiles stays on 128 x 128 tiles: 400 and K of 3072 (65536 x 512 x 4104: 609
+    //   against 766), 1024 and 1536 (8192 x 8192 x 1544 354 and 370, x 1000 252 and 241), 2048 and 512 (16384 x 8192 x
+    //   520 318 and 332);
+    // * short K and few outputs on the small-M kernel (1000 x 512 x 1024: 8.5 against 10.5; level at 32-square
+    //   tiles x K of 2^19: 500 x 2048 x 512), also with many tiles of 128 x 128 where the narrow kernel does not go
+    //   (K < 64: 1999 x 1536 x 48 8 against 15) or has little to do (100000 x 64 x 72 11 against 16) and rows are
+    //   16-byte aligned (4000 x 2047 x 48 22 against 17); from K = 2048 on only where K is no multiple of 64 and
+    //   its blocks fit one round (300 x 776 x 3472 16 and 22): its K split gives a prefix other bits than the whole.
+    const int64_t tiles256 = ((M + XBM - 1) / XBM) * ((N + XBN - 1) / XBN), tiles128 = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    const int64_t blocks = ((M + LBM - 1) / LBM) * ((N + LBN - 1) / LBN);
+    const size_t dlds = (size_t)DSTAGES * DSTAGE_BYTES;
+    bool take_dlds = g_gemm_kernel == 4;
+    const int64_t es = out_dtype == HX_BF16 ? 2 : 4;
+    const bool rows16 = (((uint64_t)(uintptr_t)Y0 | (uint64_t)(ld0 * es)) & 15) == 0 &&
+                        (split1 == N || (((uint64_t)(uintptr_t)Y1 | (uint64_t)(ld1 * es) | (uint64_t)(split1 * es)) & 15) == 0) &&
+                        (split2 == N || (((uint64_t)(uintptr_t)Y2 | (uint64_t)(ld2 * es) | (uint64_t)(split2 * es)) & 15) == 0);
+    const int64_t tiles32 = ((M + 31) / 32) * ((N + 31) / 32);
+    const bool thin = rows16 && (K < 64 || (N <= 64 && K <= 128));
+    const bool small_out = (tiles128 < 128 || thin) && (K < 2048 ? tiles32 * K <= (1 << 19) : K % 64 != 0 && tiles32 <= 256);
     if (g_gemm_kernel == 0 && vec && K % 8 == 0 && K >= 64 && !small_out) {
-        if (K % 64 == 0 && N >= 256 && M >= 256 && ((M + XBM - 1) / XBM) * ((N + XBN - 1) / XBN) >= 112 && d256_ok<64, 2>())
+        const bool whole = rows16 && M % 128 <= 32 && N % 128 <= 32 && (split1 == N || split1 % 128 == 0) &&
+                           (split2 == N || split2 % 128 == 0) && !bias && !(act & 1);
+        const bool panel = M > 128 && M <= 256 && N * K >= (1 << 25);
+        const bool panel_round = panel && N * K >= (1 << 27) && blocks <= 256;
+        if (K % 64 == 0 && N >= 256 && M >= 256 && tiles256 >= 112 && !panel_round &&
+            (rows16 ? whole || K >= 512 || tiles256 >= 160 : K >= 1024 && tiles256 >= 160) && d256_ok<64, 2>())
             return launch_d256<64, 2>(M, N, K, X, ldx, W, ldw, bias, o, stream);
+        take_dlds = K % 64 == 0 && ((K >= 2048 && blocks >= 192 && blocks <= 256) || (K >= 1024 && N > 128 && N < 256 && blocks >= 512) ||
+                                    (panel && M < 256) || panel_round);
+        const bool many = K % 64 != 0 && M >= 256 && N > 128 &&
+                          ((K >= 3072 && tiles256 >= 400) || (K >= 1536 && tiles256 >= (N < 256 ? 512 : 1024)) ||
+                           (K >= 512 && tiles256 >= 2048));
         const bool one = ((M + 63) / 64) * ((N + 127) / 128) < 160;
-        if ((N + 63) / 64 <= 65535 && (one ? narrow_ok<1>() : narrow_ok<2>()))
+        if (!(take_dlds && dlds_ok(dlds)) && !many && (N + 63) / 64 <= 65535 && (one ? narrow_ok<1>() : narrow_ok<2>()))
             return one ? launch_narrow_cb<1>(M, N, K, X, ldx, W, ldw, bias, o, stream)
                        : launch_narrow_cb<2>(M, N, K, X, ldx, W, ldw, bias, o, stream);
     }
-    const size_t dlds = (size_t)DSTAGES * DSTAGE_BYTES;
-    if (vec && K > 0 && K % LBK == 0 && g_gemm_kernel == 4 && dlds_ok(dlds)) {
+    if (vec && K > 0 && K % LBK == 0 && take_dlds && dlds_ok(dlds)) {
         dim3 lg((unsigned)((N + LBN - 1) / LBN), (unsigned)((M + LBM - 1) / LBM));
         hipLaunchKernelGGL(gemm_bf16_nt_dlds_kernel, lg, dim3(256), dlds, as_stream(stream), M, N, K,
                            (const uint16_t*)X, ldx, (const uint16_t*)W, ldw, bias, o);
         HX_LAUNCH_CHECK();
         return HX_OK;
     }
-    const int64_t tiles128 = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     if (vec && K % 8 == 0 && K >= 8 && g_gemm_kernel != 1 && g_gemm_kernel != 4 &&
         (g_gemm_kernel == 3 || tiles128 < 128 || (g_gemm_kernel == 0 && small_out)) && (M + 31) / 32 <= 65535) {
         // 64-wide tiles where they still give the GPU 256 blocks (decode in_proj), else 32-wide;

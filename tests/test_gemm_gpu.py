@@ -364,6 +364,11 @@ def test_gemm_pointer_loads_past_2gib(dev, kernel):
     (1999, 768, 1544), (1100, 1000, 1096), (64, 33000, 72),  # 128-wide
     (1792, 4096, 640), (1791, 4000, 640),                  # 112 tiles of 256 x 256 and their ragged form
     (96, 4096, 1360), (96, 4104, 1360), (33, 40, 56),      # either side of the small-M kernel's 2^19
+    (500, 500, 2056), (513, 500, 2056), (16500, 64, 72), (16500, 64, 136),  # its K from 2048 and its N up to 64
+    (1800, 4000, 448), (1800, 4000, 512), (2600, 3808, 64), (2600, 3809, 960), (2600, 3809, 1024),  # ragged 256 x 256
+    (2900, 2048, 1984), (2900, 2048, 2048), (3000, 2050, 2048),  # 256 x 128: one round of blocks,
+    (32768 * 4, 136, 1024), (130, 16384, 2048), (128, 16384, 2048), (256, 32768, 4096),  # many rows, a panel of rows
+    (5120, 5120, 3080), (5100, 5100, 1544), (8192, 8192, 1544), (65536, 512, 3080), (65536, 512, 1544),  # 128 x 128
 ])
 def test_gemm_middle_sizes(dev, M, N, K):
     """The automatic choice between one tile of 256 x 256 per CU and the small-M kernel, at its edges:
