@@ -253,17 +253,18 @@ def test_scan_segmented_long_sequence_path(dev, _reset_segments, nseg, shape, va
     assert rel_err(glast, rlast64) <= max(TOL_F32, 1.5 * rel_err(rlast, rlast64))
 
 
+@pytest.mark.parametrize("variant", [0, 42])
 @pytest.mark.parametrize("zero_a", [False, True])
-def test_scan_segmented_decay_window(dev, _reset_segments, zero_a):
+def test_scan_segmented_decay_window(dev, _reset_segments, zero_a, variant):
     """Segments long enough that the end-state pass starts late: delta_raw ~ N(0, 0.5) (dt about
     0.7) and A = -(n+1), so the decay to a 2048-step segment's end falls below 2^-32 within ~32
     steps and the end states come from that window alone (the carry takes no decay from such a
-    segment). With one state's A = 0 in one channel no window applies to that channel's wave;
-    that state then sums 8192 undamped terms, whose f32 rounding (in either summation order)
+    segment; the paired kernel, variant 0, asks after every 48 steps, for its whole block). With one
+    state's A = 0 in one channel no window applies to that channel's wave or block; that state then sums 8192 undamped terms, whose f32 rounding (in either summation order)
     exceeds the tolerance, so outputs and final state are held to the float64 restatement at the
     tolerance or 1.5x the sequential f32 oracle's own error, whichever is larger."""
     ssm.set_scan_segments(4)
-    ssm.set_scan_variant(42)
+    ssm.set_scan_variant(variant)
     x = scan_inputs(1, 8192, 64, 16, seed=0x5E6, with_bias=True)
     x["delta"] = (x["delta"] + np.float32(4.0)).astype(np.float32)
     if zero_a:
@@ -276,6 +277,10 @@ def test_scan_segmented_decay_window(dev, _reset_segments, zero_a):
           f"state: gpu {rel_err(glast, rlast64):.3e} f32 oracle {rel_err(rlast, rlast64):.3e}")
     assert rel_err(g, r64) <= max(TOL_F32, 1.5 * rel_err(r, r64))
     assert rel_err(glast, rlast64) <= max(TOL_F32, 1.5 * rel_err(rlast, rlast64))
+    # the window is applied, and only there: a NaN before it leaves the next segment finite, unless A = 0 keeps it
+    x["u"][0, 100, 5] = np.nan
+    late = run_gpu(x, dev)[0, 2048:, 5]
+    assert not np.isfinite(late).any() if zero_a else np.isfinite(late).all()
 
 
 @pytest.mark.parametrize("variant", [0, 40, 42])
@@ -370,6 +375,30 @@ def test_scan_dtproj_matches_separate_steps(dev, bt, L, dim, r):
     assert e_sep <= 4e-3 and e_ref <= 1e-2, (e_sep, e_ref)
 
 
+def test_scan_paired_kernel_stores_near_its_largest_offset(dev):
+    """A partial last tile in a batch row just below 2^31 bytes (1 x 53585 x 10001 fp32, 2.14 GB per operand): the
+    lanes of channels past dim, and the steps past the end, are dropped, also where a row's offset is added to the
+    offset that drops them. Every element is written once (rows are compared with the same channels alone), and
+    nothing before or after the output."""
+    L, dim = 53585, 10001
+    assert (L + 96) * dim * 4 < 2 ** 31 <= (L + 97) * dim * 4  # the longest that it takes
+    g = torch.Generator(device=dev).manual_seed(3)
+    u = torch.randn((1, L, dim), generator=g, device=dev)
+    delta = torch.randn((1, L, dim), generator=g, device=dev) * 0.5 - 4.0
+    B, C = (torch.randn((1, L, 16), generator=g, device=dev) for _ in range(2))
+    A, D = -torch.arange(1.0, 17.0, device=dev).repeat(dim, 1), torch.randn(dim, generator=g, device=dev)
+    buf = torch.full((L * dim + 2 * 4096,), float("nan"), device=dev)
+    out = buf[4096:-4096].view(1, L, dim)
+    ssm.selective_scan_fwd(u, delta, A, B, C, D, out=out)
+    torch.cuda.synchronize()
+    assert torch.isnan(buf[:4096]).all() and torch.isnan(buf[-4096:]).all()
+    assert int(torch.isnan(out).sum()) == 0
+    for c0, c1 in ((0, 64), (dim - 17, dim)):  # the first tile and the partial one
+        part = ssm.selective_scan_fwd(*(t[..., c0:c1].contiguous() for t in (u, delta)), A[c0:c1].contiguous(), B, C,
+                                      D[c0:c1].contiguous())
+        assert norm_err(part.cpu(), out[..., c0:c1].cpu()) <= TOL_F32
+
+
 @pytest.mark.parametrize("bt,L,dim,r", [(1024, 16, 64, 32), (1024, 48, 60, 128), (2048, 96, 64, 64), (1024, 49, 64, 96)])
 def test_scan_dtproj_many_short_sequences(dev, bt, L, dim, r):
     """Too many short sequences for the paired kernel's read-ahead take the wave kernel, with the same bits as a few
@@ -425,23 +454,33 @@ def test_scan_dtproj_errors_and_empty(dev):
 
 
 @pytest.mark.parametrize("with_z", [True, False])
-@pytest.mark.parametrize("bt,L,dim", [(1, 1, 4), (2, 15, 68), (3, 16, 64), (2, 17, 60), (1, 47, 128), (2, 48, 192),
-                                      (2, 49, 132), (1, 97, 1000), (5, 250, 64)])
-def test_scan_paired_kernel_matches_wave_kernel_bitwise(dev, bt, L, dim, with_z):
-    """bf16's automatic kernel (state and element waves in pairs) performs the wave kernel's (42)
+@pytest.mark.parametrize("bt,L,dim,dtype,scale", [
+    (1, 1, 4, "bf16", 1), (2, 15, 68, "bf16", 1), (3, 16, 64, "bf16", 1), (2, 17, 60, "bf16", 1), (1, 47, 128, "bf16", 1),
+    (2, 48, 192, "bf16", 1), (2, 49, 132, "bf16", 1), (1, 97, 1000, "bf16", 1), (5, 250, 64, "bf16", 1),
+    (260, 17, 48, "f32", 1), (260, 49, 36, "f32", 1), (130, 250, 68, "f32", 1),  # more than one 48-channel group per CU
+    (2, 49, 132, "bf16", 1e-20), (260, 49, 36, "f32", 1e-20)])  # inputs B * (dt*u) below 2^-126
+def test_scan_paired_kernel_matches_wave_kernel_bitwise(dev, bt, L, dim, dtype, scale, with_z):
+    """The automatic kernel (state and element waves in pairs) performs the wave kernel's (42)
     operations in its order: the same bits around its edges, 16-step chunks in rounds of three and
-    64-channel tiles, with an initial state and the final state."""
+    64-channel tiles, with an initial state and the final state, for subnormal products too (the matrix
+    core forms them)."""
     x = scan_inputs(bt, L, dim, 16, seed=L * 7 + dim, with_z=with_z, with_bias=True)
-    init = (np.random.default_rng(L).standard_normal((bt, dim, 16)) * 0.5).astype(np.float32)
+    x["u"], x["B"] = x["u"] * np.float32(scale), x["B"] * np.float32(scale)
+    init = (np.random.default_rng(L).standard_normal((bt, dim, 16)) * 0.5 * scale ** 2).astype(np.float32)
+    if scale != 1:
+        x["D"] = None  # outputs of the states alone
+    kw = dict(dtype=torch.bfloat16 if dtype == "bf16" else torch.float32, init_state=init, last=True)
     ssm.set_scan_segments(1)
     try:
-        auto = run_gpu(x, dev, dtype=torch.bfloat16, init_state=init, last=True)
+        auto = run_gpu(x, dev, **kw)
         ssm.set_scan_variant(42)
-        wave = run_gpu(x, dev, dtype=torch.bfloat16, init_state=init, last=True)
+        wave = run_gpu(x, dev, **kw)
     finally:
         ssm.set_scan_segments(0)
     assert np.array_equal(auto[0], wave[0])
     assert np.array_equal(auto[1], wave[1])
+    if scale != 1:
+        assert (auto[1] != 0).mean() > 0.9 and np.abs(auto[1]).max() < 2.0 ** -126
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
