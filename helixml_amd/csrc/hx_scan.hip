@@ -1731,7 +1731,7 @@ struct ScanArgs {
     const float* init_state;
     float* last_state;
     hipStream_t stream;
-    void* ws = nullptr;      // caller workspace for the segmented long-sequence path (nullable:
+    void* ws = nullptr;      // caller workspace for cutting the sequence into segments (nullable:
     size_t ws_bytes = 0;     // without one the sequence is never segmented)
     bool ws_may_be_short = false;  // the workspace is a buffer that happens to be free: use what fits
 };
@@ -2286,11 +2286,11 @@ extern "C" int hx_selective_scan_fwd_ws(int64_t batch, int64_t seqlen, int64_t d
 }
 
 // ------------------------------------------------------------------ no-allocation entry point
-// Scratch of hx_selective_scan_fwd_noalloc: the segmented long-sequence path's end states, entry
-// states and segment decays (the same layout a caller workspace holds for
-// hx_selective_scan_fwd_ws). One copy per device, resident until the process ends. Nothing in it
-// has to start at zero: the end-state pass writes every end state and decay the carry kernel
-// reads, and the carry kernel writes every entry state the output pass reads.
+// Scratch of hx_selective_scan_fwd_noalloc: end states and decays of a cut sequence's segments, and the
+// wave path's entry states (the same layout a caller workspace holds for hx_selective_scan_fwd_ws). The
+// automatic kernel needs at most 4 MB of it, two blocks per CU. One copy per device, resident until the
+// process ends. Nothing in it has to start at zero: the end-state pass writes every end state and decay
+// that is read after it.
 constexpr size_t kScanScratchBytes = (size_t)8 << 20;
 static __device__ __align__(256) unsigned char scratch[kScanScratchBytes];
 

@@ -61,10 +61,10 @@ __device__ inline float to_f32(uint16_t v) { return bf16_bits_to_f32(v); }
 // Every operation is scan_wave3_kernel's in its order, so results match it bit for bit.
 //
 // Bound: instruction issue. The state wave is the critical path, 18 instructions a step at the 5-6
-// cycles (10 for exp2) that one wave takes for each; the SIMD's VALU is 70-75% busy over both waves,
-// 25% fewer VALU cycles than scan_ws2_kernel at the same shape. Measured (gfx950): 16 x 8192 x 1024 bf16 with rank 32
-// 666 -> 540 us, 4 x 4096 x 4096 with rank 128 338 -> 275 us (scan_wave3_kernel, one wave a SIMD);
-// 1 x 65536 x 2048 fp32, segmented, 686 -> 590 us. Splitting the states over two waves (three waves
+// cycles (10 for exp2) that one wave takes for each; the SIMD's VALU is 73-77% busy over both waves with one
+// block per CU (88% with two), 25% fewer VALU cycles than scan_ws2_kernel at the same shape. Measured (gfx950):
+// 16 x 8192 x 1024 bf16 with rank 32 666 -> 540 us, 4 x 4096 x 4096 with rank 128 338 -> 285 us (scan_wave3_kernel,
+// one wave a SIMD); 1 x 65536 x 2048 fp32, segmented, 695 -> 603 us. Splitting the states over two waves (three waves
 // a SIMD) was slower, 600 us at the first shape: readouts and hand-over double. The state waves'
 // priority gives 2-3%.
 //

@@ -442,7 +442,7 @@ MemoryHandle RocmBackend::execute_op(const Operation& op) {
             return o;
         }
         case OperationType::SSMForward: {
-            // the library's long-sequence path (time segments with a carry) through a workspace
+            // the library cuts sequences of few channels into time segments, through a workspace
             // this backend keeps, as the fused scan of hal/src/device.rs:191 would run
             const int64_t bt = (int64_t)param("batch", 0), L = (int64_t)param("seqlen", 0);
             const int64_t dim = (int64_t)param("dim", 0), N = (int64_t)param("dstate", 16);

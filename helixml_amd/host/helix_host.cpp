@@ -381,7 +381,7 @@ HipTensor selective_scan(const HipTensor& u, const HipTensor& delta, const HipTe
     HipTensor out(u.shape(), u.storage(), 0);
     if (last_state) *last_state = HipTensor(Shape({bt, dim, N}), Storage::F32, 0);
     const int dt = u.storage() == Storage::BF16 ? HX_BF16 : HX_F32;
-    // the long-sequence path (time segments with a carry) needs scratch: kept per thread and
+    // cutting a sequence into time segments needs scratch: kept per thread and
     // grown on demand (this thread's calls are ordered on the default stream, so they share it)
     thread_local HipTensor ws;
     const size_t need = hx_selective_scan_workspace_size((int64_t)bt, (int64_t)L, (int64_t)dim, (int64_t)N, dt);

@@ -88,8 +88,8 @@ def selective_scan_fwd(u, delta, A, B, C, D=None, z=None, dt_bias=None, delta_so
                        stream=None):
     """Fused selective scan (hx_selective_scan_fwd_ws). u, delta, z: [batch, L, dim];
     B, C: [batch, L, dstate]; A: [dim, dstate] fp32; D, dt_bias: [dim] fp32. ``workspace``: a
-    uint8 device tensor of at least selective_scan_workspace_size(...) bytes for the segmented
-    long-sequence path; allocated here (by torch, outside the library) when not given."""
+    uint8 device tensor of at least selective_scan_workspace_size(...) bytes for the time segments
+    of few channels; allocated here (by torch, outside the library) when not given."""
     if u.dim() != 3:
         raise ShapeMismatch(f"u: expected 3 dims [batch, seqlen, dim], got {list(u.shape)}")
     bt, L, dim = u.shape

@@ -522,7 +522,7 @@ public:
     void synchronize() override;
 
 private:
-    // device scratch of the scan's long-sequence path, kept between SSMForward operations and
+    // device scratch of the scan's time segments, kept between SSMForward operations and
     // grown on demand (operations of one backend run in order on the default stream)
     void* scan_workspace(size_t bytes);
     int device_;

@@ -7,7 +7,7 @@
  * enums: no HIP, torch or C++ types cross it. Inputs and outputs are allocated by the caller
  * (hx_malloc, or any HIP allocation on the same device). No compute entry point allocates:
  * scratch memory is a caller-owned workspace whose size the matching *_workspace_size function
- * returns (the block and layer forwards, the long-sequence scan, the S4 paths).
+ * returns (the block and layer forwards, the segmented scan, the S4 paths).
  * A `stream` argument is a hipStream_t passed as void*
  * (NULL = the legacy default stream). All compute entry points are stream-ordered and
  * asynchronous; they validate shapes on the host before any launch and return a status code.
@@ -123,8 +123,9 @@ int hx_selective_scan_fwd_ws(int64_t batch, int64_t seqlen, int64_t dim, int64_t
                              void* workspace, size_t workspace_bytes, void* stream);
 
 /* hx_selective_scan_fwd_ws without the workspace argument, for callers that cannot allocate
- * (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc): the segmented
- * long-sequence path uses an 8 MiB device-resident scratch array of the library instead (one per
+ * (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc): sequences that are
+ * cut into segments (hx_selective_scan_workspace_size > 0: few channels and at least 512 steps) use an
+ * 8 MiB device-resident scratch array of the library instead (one per
  * device, held until the process ends; hx_init or the first call on a device resolves its
  * address). Calls nothing that allocates. Shapes whose segmented path needs more than 8 MiB
  * (hx_selective_scan_workspace_size > 8 MiB, e.g. with hx_set_scan_segments forcing thousands of
@@ -399,8 +400,9 @@ int hx_set_scan_variant(int variant);
  * kernel: 64-row tiles holding every column (N <= 256, K % 64 == 0), 8 the persistent form of 5
  * (one block per CU walks its tiles, the K-tile ring runs on across them; same bits as 5; the
  * automatic choice where K <= 1024 and there are at least two tiles per CU). The automatic choice also
- * takes products of middle size through the narrow kernel over a grid of column tiles. A shape a forced kernel cannot take goes to the 128x128 kernel (the
- * small-M one for small shapes). A measurement knob. */
+ * takes products of middle size through the narrow kernel over a grid of column tiles. A shape a
+ * forced kernel cannot take goes to the 128x128 kernel (the small-M one for small shapes). A
+ * measurement knob. */
 int hx_set_gemm_kernel(int k);
 /* S4D knobs for later calls on the calling thread: path 0 auto (wave path for dstate 16), 1 the
  * per-channel thread path; time segments 0 auto, n forced. */
