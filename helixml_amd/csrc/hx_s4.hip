@@ -1422,7 +1422,8 @@ int launch_s4d_wave(int64_t Bt, int64_t L, int64_t Dm, const float* x, const flo
         nseg = (L + seg_len - 1) / seg_len;
     }
     HX_REQUIRE(pairs * nseg <= 0x7fffffff, HX_ERR_UNSUPPORTED, "s4d_complex: grid too large");
-    const S4dSeg sg{seg_len, (int)nseg, whole, scratch};
+    // segments below 512 steps hardly reach the decay that lets them start late
+    const S4dSeg sg{seg_len, (int)nseg, whole || (seg_len < 512 && g_s4d_segments <= 0), scratch};
     auto run = [&](auto kernel, int64_t segs) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)(pairs * segs)), dim3(256), 0, s, L, Dm, ntiles, Bt, x, dt,
                            a_re, a_im, B_re, B_im, C_re, C_im, D, y, sg);

@@ -1805,10 +1805,10 @@ bool tile_ok(const ScanArgs& a) {
 }
 size_t wave_workspace_bytes(const ScanArgs& a, size_t es);
 // Sequences given with a workspace may leave out what has decayed below kDecayDrop from this length on,
-// where the wave path cuts them too: at dt near 0.02 the end-state pass of 65536 steps then walks about 1100
-// of each segment's 4096. Shorter segments hardly reach that decay. All others walk whole segments, so that
-// a NaN, an infinity or an outlier reaches everything after it.
-constexpr int64_t kDropSteps = 4096;
+// where the wave path cuts them too, and in segments as long as its own: at dt near 0.02 the end-state pass of
+// 65536 steps then walks about 1100 of each segment's 4096. Shorter segments hardly reach that decay. All others
+// walk whole segments, so that a NaN, an infinity or an outlier reaches everything after it.
+constexpr int64_t kDropSteps = 4096, kDropSegment = 1024;
 bool ps_drop(const ScanArgs& a, size_t es) {
     return a.L >= kDropSteps && !a.ws_may_be_short && wave_workspace_bytes(a, es) > 0;
 }
@@ -1853,7 +1853,7 @@ int launch_ps(const ScanArgs& a, const uint16_t* dtlo, const uint16_t* wdt) {
     float4* hend = (float4*)a.ws;
     float4* decay = hend + (nseg - 1) * a.Bt * ntiles * 256;
     const PsArgs pa{a.L, a.Dm, (int)ntiles, (int)a.Bt, (int)nseg, (int)seg_len,
-                    drop, a.A, a.D, a.dt_bias,
+                    drop && (seg_len >= kDropSegment || g_scan_segments > 0), a.A, a.D, a.dt_bias,
                     a.init_state, a.last_state, hend, decay, dtlo, wdt};
     if (nseg > 1) {
         hipLaunchKernelGGL((scan_ps_kernel<T, false, SP, true, DTPK>), dim3((unsigned)(ntiles * a.Bt * (nseg - 1))),

@@ -73,8 +73,8 @@ __device__ inline float to_f32(uint16_t v) { return bf16_bits_to_f32(v); }
 // (a sum per state, one FMA each: A = -inf gives S = -inf, where A times a sum of dt would be NaN at the last
 // step, whose sum is 0), and stops at the first 48-step round at which every state of the block's channels has decayed
 // below 2^-32 (kDecayDrop): what is left out is 2^-8 of the fp32 rounding of the state there. Such a
-// segment publishes decay 0. Below 4096 steps, in the Mamba block, and for dims that are no multiple of 4
-// or rows that are not 16-byte aligned (drop = 0) it walks its whole segment instead: a NaN, an infinity or
+// segment publishes decay 0. Below 4096 steps, in segments below 1024, in the Mamba block, and for dims that are no
+// multiple of 4 or rows that are not 16-byte aligned (drop = 0) it walks its whole segment instead: a NaN, an infinity or
 // an outlier reaches everything after it, as in the uncut scan, and segments of a few hundred steps hardly
 // ever decay that far. The output pass chains the segments before its own itself.
 // Sizes: byte offsets inside a segment below 2^31, in B and C (16 wide) too.

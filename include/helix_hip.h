@@ -104,9 +104,9 @@ int hx_selective_scan_fwd(int64_t batch, int64_t seqlen, int64_t dim, int64_t ds
  * cut into time segments whose end states (from a zero state) are accumulated backwards from
  * each segment's end, and every segment is then scanned with outputs from the chained entry state
  * (results agree with the unsegmented scan to fp32 rounding). From 4096 steps on, with dim % 4 == 0 and
- * 16-byte aligned rows, fewer than 256 (batch, 64-channel) tiles, the accumulation stops once every
- * state's decay to the segment's end is below 2^-32, which leaves out what came before (a NaN included);
- * elsewhere it walks whole segments. workspace: device memory of at least
+ * 16-byte aligned rows, fewer than 256 (batch, 64-channel) tiles and segments of at least 1024 steps, the
+ * accumulation stops once every state's decay to the segment's end is below 2^-32, which leaves out what
+ * came before (a NaN included); elsewhere it walks whole segments. workspace: device memory of at least
  * hx_selective_scan_workspace_size(...) bytes, 16-byte aligned (0 bytes: no segments); it holds no state
  * between calls. With fewer bytes as many segments as fit are used, except that those sequences of
  * 4096 steps and more refuse a workspace below min(512 / tiles rounded up, seqlen / 1024) segments of
@@ -197,7 +197,11 @@ int hx_s4_ref_fwd_parallel(int64_t d_model, int64_t dstate, int64_t seqlen, floa
  *   h[d,n] = Abar*h + Bbar*x[b,t,d];  y[b,t,d] = 2*Re(sum_n C[d,n]*h[d,n]) + D[d]*x[b,t,d]
  * x, y: [batch, seqlen, dim] fp32. a_re, a_im, B_re, B_im, C_re, C_im: [dim, dstate]; dt, D: [dim].
  * workspace: at least hx_s4d_workspace_size(...) bytes (segment states; 0 when the sequence is not
- * segmented), 16-byte aligned. */
+ * segmented), 16-byte aligned; with fewer as many segments as fit are used, except that sequences of 1024
+ * steps and more with dim % 4 == 0 and 16-byte aligned rows refuse a workspace below the states of
+ * 2 * min(512 / tiles rounded up, seqlen / 512) segments (a count of 1 needs none). Those sequences leave
+ * out, where their segments are at least 512 steps long, what has decayed below 2^-32 at a segment's end (a
+ * NaN included). */
 size_t hx_s4d_workspace_size(int64_t batch, int64_t seqlen, int64_t dim, int64_t dstate);
 int hx_s4d_complex_fwd(int64_t batch, int64_t seqlen, int64_t dim, int64_t dstate,
                        const float* x, const float* dt,

@@ -231,16 +231,21 @@ def test_s4d_wave_path(dev, bt, L, dim, nseg):
 def test_s4d_automatic_segments(dev, bt, L, dim):
     """Sequences of few channels are cut by themselves, on both sides of the shortest that is (320 steps), with
     ragged last segments and channel tiles; without a workspace they stay whole where none was ever
-    needed (below 1024 steps). A NaN reaches every later output of its channel and no other's."""
+    needed (below 1024 steps). A NaN reaches every later output of its channel and no other's, also from 1024
+    steps on while segments are shorter than 512 steps."""
     x, p = s4d_inputs(bt, L, dim, 16, seed=L + dim)
     kw = {k: dv(v, dev) for k, v in p.items()}
     r = oracle.s4d_complex(x, **p)
     from helixml_amd import _ffi
     assert (_ffi.lib().hx_s4d_workspace_size(bt, L, dim, 16) > 0) == (L >= 320)
     assert rel_err(ssm.s4d_complex_fwd(dv(x, dev), **kw).cpu().numpy(), r) <= TOL_F32
-    if L >= 1024:
-        return
     xd = dv(x, dev)
+    if L >= 1024:
+        kw["a_re"] = kw["a_re"] * 20
+        xd[0, 2, 0] = float("nan")
+        bad = torch.isnan(ssm.s4d_complex_fwd(xd, **kw)).cpu().numpy()
+        assert bad[0, 2:, 0].all() and bad.sum() == L - 2
+        return
     y = torch.full_like(xd, float("nan"))
     _ffi.call("hx_s4d_complex_fwd", bt, L, dim, 16, xd.data_ptr(),
               *[kw[k].data_ptr() for k in ("dt", "a_re", "a_im", "B_re", "B_im", "C_re", "C_im", "D")],

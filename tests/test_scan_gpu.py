@@ -550,10 +550,11 @@ def test_scan_workspace_below_the_size_asked_for(dev):
 
 
 @pytest.mark.parametrize("value", [float("nan"), float("inf"), 1e30])
-@pytest.mark.parametrize("L,dim,offset", [(1000, 64, 0), (8192, 62, 0), (8192, 65, 0), (8192, 64, 1)])
+@pytest.mark.parametrize("L,dim,offset", [(1000, 64, 0), (8192, 62, 0), (8192, 65, 0), (8192, 64, 1), (8192, 64, 0)])
 def test_scan_automatic_segments_keep_non_finite_values(dev, value, L, dim, offset):
     """A sequence below 4096 steps that is cut by itself loses no NaN, infinity or outlier, nor does one of any length
-    whose dim is no multiple of 4 or whose rows are not 16-byte aligned: one input early in the first segment, with
+    whose dim is no multiple of 4 or whose rows are not 16-byte aligned, or whose segments are shorter than the wave
+    path's 1024 steps: one input early in the first segment, with
     steps so large that its state decays below 2^-32 before that segment ends. A NaN or an infinity leaves that
     channel's later outputs without a finite value, as the recurrence does, and no other channel's; the outlier's
     state, exp(-0.6 * 94) of it by then, still dominates the next segment (float64: steps 96 to 111). That decay's
