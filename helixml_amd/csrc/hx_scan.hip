@@ -1823,10 +1823,12 @@ bool ps_ok(int64_t Bt, int64_t Dm, int64_t L, size_t es) {
 // step, which a few steps do not pay for; the wave kernels keep more blocks in flight. us, paired against wave
 // kernel (the same bits): 4096 tiles x 1 step 33 and 25, x 32 45 and 40, x 96 bf16 102 and 99, x 128 128 and 130;
 // 1024 tiles x 16 10.8 and 9.5, x 48 18.7 and 18.0, x 64 21.5 and 22.2; with the fused dt projection (rank 128)
-// 4096 tiles x 16 58 and 41, x 64 95 and 85. At 512 tiles they are level.
-bool ps_brief(int64_t Bt, int64_t Dm, int64_t L) {
+// 4096 tiles x 16 58 and 41, x 64 95 and 85. Past one round of blocks a single chunk is enough (800 tiles x 8
+// fp32 10.9 and 9.5); up to there they are level, but for the kernels with dt_proj (16 tiles x 16, rank 128, 6.6
+// and 5.6; 512 x 16 10.5 and 8.6) and the fast kernel (16 tiles x 16 4.8 and 4.0; 512 x 16 7.1 and 6.0): chunk.
+bool ps_brief(int64_t Bt, int64_t Dm, int64_t L, bool chunk) {
     const int64_t tiles = Bt * ((Dm + 63) / 64), cus = device_cus();
-    return tiles >= 4 * cus && L <= (tiles >= 8 * cus ? 96 : 48);
+    return L <= (tiles >= 8 * cus ? 96 : tiles >= 4 * cus ? 48 : tiles > 2 * cus || chunk ? 16 : 0);
 }
 
 template <typename T, bool HAS_Z, bool SP, int DTPK>
@@ -2072,7 +2074,7 @@ int run_scan(const ScanArgs& a) {
         // and sizes past the paired kernel's offsets take the wave kernels where their float4 access is legal, and
         // otherwise the fast kernel, which leads for one chunk (1536 tiles x 16 steps 11.5 us against 15, x 32 20
         // against 19)
-        if (ps_ok(a.Bt, a.Dm, a.L, es) && !(ps_brief(a.Bt, a.Dm, a.L) && (tiles || a.L <= 16))) {
+        if (ps_ok(a.Bt, a.Dm, a.L, es) && !(ps_brief(a.Bt, a.Dm, a.L, !tiles) && (tiles || a.L <= 16))) {
             const bool cut = a.ws && ps_segments(a.Bt, a.Dm, a.L, ps_drop(a, es)) > 1;
             if constexpr (std::is_same<T, float>::value)
                 if (!cut && tiles && ws2_ok<T>(a) && a.Bt * ((a.Dm + 47) / 48) <= device_cus())
@@ -2207,7 +2209,7 @@ int scan_fwd_dtproj(int64_t batch, int64_t seqlen, int64_t dim, const uint16_t* 
     HX_REQUIRE(aligned(u, 16) && aligned(z, 16) && aligned(out, 16) && aligned(dtlo, 16) && aligned(w_dt, 16) &&
                    aligned(B, 32) && aligned(C, 32) && (!D || aligned(D, 16)) && (!dt_bias || aligned(dt_bias, 16)),
                HX_ERR_UNSUPPORTED, "selective scan with dt_proj: operands not 16-byte aligned");
-    if (ps_ok(batch, dim, seqlen, 2) && !ps_brief(batch, dim, seqlen)) {
+    if (ps_ok(batch, dim, seqlen, 2) && !ps_brief(batch, dim, seqlen, true)) {
         const ScanArgs a{batch, seqlen, dim, 16, 1, u, nullptr, A, B, C, D, z, dt_bias, out, nullptr, last_state,
                          stream, ws, ws_bytes, true};
         switch (rank / 32) {

@@ -331,7 +331,8 @@ def test_warp_specialised_partial_group_large_offsets(dev, variant):
 
 
 @pytest.mark.parametrize("bt,L,dim,r", [(2, 37, 256, 32), (1, 130, 128, 64), (3, 50, 192, 96),
-                                        (1, 33, 256, 128), (2, 1000, 64, 32)])
+                                        (1, 33, 256, 128), (2, 1000, 64, 32),
+                                        (2, 16, 256, 32), (1, 9, 132, 128), (3, 17, 64, 64)])  # one chunk and one step more
 def test_scan_dtproj_matches_separate_steps(dev, bt, L, dim, r):
     """hx_selective_scan_dtproj_fwd against the block's two separate steps, dt = gemm_bf16(dt_lo,
     w_dt) then the wave kernel (variant 42, whose arithmetic the fused kernel shares): the two
@@ -485,9 +486,10 @@ def test_scan_paired_kernel_matches_wave_kernel_bitwise(dev, bt, L, dim, dtype, 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("bt,L,dim", [(1023, 48, 60), (1024, 1, 64), (1024, 48, 60), (1024, 49, 64), (2048, 96, 4),
-                                      (2048, 97, 8), (1024, 16, 62), (1024, 17, 62)])
+                                      (2048, 97, 8), (1024, 16, 62), (1024, 17, 62), (513, 16, 64), (512, 16, 64),
+                                      (513, 17, 64), (2, 16, 130), (2, 17, 130), (3, 5, 63)])
 def test_scan_many_short_sequences(dev, bt, L, dim, dtype):
-    """Either side of the sizes whose short sequences are too many for the paired kernel's read-ahead: rows of
+    """Either side of the sizes whose short sequences do not pay for the paired kernel's read-ahead: rows of
     16-byte pieces give the wave kernel's bits whichever kernel takes them, the others agree with the float64
     restatement, with an initial state and the final state."""
     x = scan_inputs(bt, L, dim, 16, seed=L * 7 + dim, with_bias=True)
